@@ -143,3 +143,50 @@ def test_device_derham_matrices_match_oracle(ctx, shell):
     with pytest.raises((LfrError, KeyError)):
         api.compute_derham_matrices({k: v for k, v in t.items() if k != "basis_w1"}, chi_f, sp,
                                     outputs=("grad",))
+
+
+@pytest.mark.parametrize("nl", [1, 3])
+@pytest.mark.parametrize("broken", ["same", "scaled"])
+def test_derham_shared_jacobian_equals_single_forms(ctx, nl, broken):
+    """The shared-Jacobian kernels (tables with the lowest-order structure)
+    against the single-form kernels on the same tables: a component of 1e-300
+    off a function's axis changes no result but leaves that structure.
+    864 nl cell-layers is not a whole number of waves.  Both sum 27 products
+    of a few rounded factors an entry, so they agree to 1e-13 of the largest
+    entry, as each does with the oracle."""
+    from lfric_core_amd import api
+    print(f"case derham shared against single nl={nl} broken={broken}", flush=True)
+    g = np.load(GOLDEN / "meshes.npz")
+    chi = shell_corners(g["C12_node_x"], g["C12_node_y"], g["C12_face_nodes"], 6.371e6,
+                        np.linspace(0.0, 2.0e4, nl + 1))
+    fs = build_dofmap(cubed_sphere(12), "W0", nl)
+    d = np.load(GOLDEN / "fs_test_data.npz")
+    _, w = gauss_rule(3)
+    t = _derham_tables(d, np.outer(w, w).ravel(), w)
+    if broken == "scaled":
+        t["basis_w2b"] = 0.5 * t["basis_w2b"]
+    off = dict(t)
+    for name, c, df in (("basis_w1", 0, 0), ("basis_w2", 2, 1), ("basis_w2b", 0, 4)):
+        off[name] = t[name].copy()
+        assert off[name][c, df, 4, 1] == 0.0
+        off[name][c, df, 4, 1] = 1e-300
+    sp = api.Space(ctx, fs)
+    chi_f = torch.from_numpy(w0_chi_fields(fs, chi)).to(ctx.device)
+    a = api.compute_derham_matrices(t, chi_f, sp)
+    b = api.compute_derham_matrices(off, chi_f, sp)
+    torch.cuda.synchronize()
+    for name in a:
+        x, y = a[name].cpu().numpy(), b[name].cpu().numpy()
+        assert np.abs(x - y).max() <= 1e-13 * np.abs(y).max(), name
+    # each output by itself has the bits of the call that makes all of them
+    for name in a:
+        one = api.compute_derham_matrices(t, chi_f, sp, outputs=(name,))
+        assert torch.equal(one[name], a[name]), name
+    # a curl (grad) table that is not the complex's leaves only that form
+    wrong = dict(t, diff_basis_w1=2.0 * t["diff_basis_w1"], diff_basis_w0=-t["diff_basis_w0"])
+    c = api.compute_derham_matrices(wrong, chi_f, sp, outputs=("mm1", "mm2", "grad", "curl"))
+    torch.cuda.synchronize()
+    assert torch.equal(c["mm1"], a["mm1"]) and torch.equal(c["mm2"], a["mm2"])
+    for name, f in (("curl", 2.0), ("grad", -1.0)):
+        x, y = c[name].cpu().numpy(), f * a[name].cpu().numpy()
+        assert np.abs(x - y).max() <= 1e-13 * np.abs(y).max(), name
