@@ -10,16 +10,13 @@
 // = (sub, diag, super); one reciprocal of the pivot per row, then the products
 // inv*c and inv*(x - a*d') exactly as written there.
 //
-// Mapping: one lane per column, 64 columns per workgroup.  A lane reads its
-// column's bands (contiguous in columnwise_matrix(bw, nrow, ncell)) and
-// right-hand side straight from global memory, every load a constant offset
-// from one per-lane base, issued kPf rows ahead of the recurrence (rows are
-// unrolled, NROW a compile-time constant, and scheduling barriers keep each
-// group of loads one group ahead); c' goes to LDS, d' stays in registers,
-// and the solution goes back through LDS for a coalesced store.
+// FP32 columns of 70 rows (W3 at 70 layers) have kernels that load a whole
+// column up front (k_appinv_deep); every other row count and kind runs
+// k_thomas_rows, which stages its loads ahead of the recurrence.
 #include <algorithm>
 #include <cmath>
 #include <cstdint>
+#include <type_traits>
 #include <vector>
 
 #include "lfr_internal.h"
@@ -28,7 +25,6 @@ namespace {
 
 constexpr int kCols = 64;   // columns (lanes) per workgroup
 constexpr int kCh = 14;     // rows per LDS stage of the solution store
-constexpr int kPf = 10;     // rows of loads ahead of a column recurrence (<= 63 loads in flight)
 
 // indirection_dofmap(i) - 1, clamped into the column's rows 0..nrow-1 so that
 // no access leaves the column (lfr_cma_create validates its maps; the raw
@@ -38,97 +34,12 @@ __device__ __forceinline__ int ind0(const int32_t* __restrict__ ind, int i, int 
   return v < 0 ? 0 : (v >= nrow ? nrow - 1 : v);
 }
 
-template <typename T, typename C, int NROW>
-__global__ void __launch_bounds__(kCols)
-k_appinv(T* __restrict__ lhs, const T* __restrict__ x, const T* __restrict__ cm,
-         const int32_t* __restrict__ map0, int ndf, const int32_t* __restrict__ ind,
-         int ncell) {
-  constexpr int NST = (NROW + kCh - 1) / kCh;
-  constexpr int PITCH_X = kCh + 1;         // odd pitch: conflict-free lane-strided access
-  __shared__ T sx[kCols * PITCH_X];
-  __shared__ int32_t sbase[kCols];
-  __shared__ int32_t sind[NROW];   // indirection_dofmap - 1, read once
-  constexpr int PC = NROW | 1;     // odd pitch of the c' rows
-  __shared__ C scp[kCols * PC];    // c' of every lane's column (registers hold d')
-  const int lane = threadIdx.x;
-  const int c0 = blockIdx.x * kCols;
-  const int ncols = min(kCols, ncell - c0);
-  if (lane < ncols) sbase[lane] = map0[(int64_t)(c0 + lane) * ndf];
-  for (int i = lane; i < NROW; i += kCols) sind[i] = ind0(ind, i, NROW);
-  C* cp = scp + lane * PC;
-  C dp[NROW];
-  // forward sweep straight from global memory: lane = column, its bands
-  // are contiguous (3 NROW values) and so are its W3 dofs, so each load is a
-  // constant offset from one per-lane base.  Loads run kPf rows ahead of the
-  // recurrence: scheduling region r holds the loads of rows [r kPf, (r+1) kPf)
-  // and the recurrence of the kPf rows before them, and no instruction
-  // crosses a region boundary, so about 4 kPf loads are in flight while the
-  // recurrence runs (a partial last workgroup clamps idle lanes to a real
-  // column).
-  {
-    const int cl = min(lane, ncols - 1);
-    const T* mb = cm + (int64_t)(c0 + cl) * 3 * NROW;
-    const T* xb = x + map0[(int64_t)(c0 + cl) * ndf];
-    T la[NROW], ld[NROW], lu[NROW], lx[NROW];
-#pragma unroll
-    for (int t = 0; t < NROW + kPf; ++t) {
-      if (t < NROW) {
-        la[t] = mb[3 * t + 0];
-        ld[t] = mb[3 * t + 1];
-        lu[t] = mb[3 * t + 2];
-        lx[t] = xb[ind0(ind, t, NROW)];
-      }
-      if (t >= kPf) {
-        const int i = t - kPf;
-        const C a = (C)la[i], d = (C)ld[i], u = (C)lu[i], xv = (C)lx[i];
-        if (i == 0) {
-          const C inv = C(1) / d;
-          cp[i] = inv * u;
-          dp[i] = inv * xv;
-        } else {
-          const C ac = a * cp[i - 1];
-          const C inv = C(1) / (d - ac);
-          if (i < NROW - 1) cp[i] = inv * u;
-          const C ad = a * dp[i - 1];
-          dp[i] = inv * (xv - ad);
-        }
-      }
-      if ((t + 1) % kPf == 0) __builtin_amdgcn_sched_barrier(0);
-    }
-  }
-  // backward substitution in registers
-#pragma unroll
-  for (int i = NROW - 2; i >= 0; --i) {
-    const C cd = cp[i] * dp[i + 1];
-    dp[i] = dp[i] - cd;
-  }
-  // stage the solution back through LDS for the store
-#pragma unroll
-  for (int s = 0; s < NST; ++s) {
-    const int r0 = s * kCh;
-    const int nr = (NROW - r0) < kCh ? (NROW - r0) : kCh;
-    __syncthreads();
-    if (lane < ncols) {
-#pragma unroll
-      for (int q = 0; q < kCh; ++q)
-        if (r0 + q < NROW) sx[lane * PITCH_X + q] = (T)dp[r0 + q];
-    }
-    __syncthreads();
-    const int nx = ncols * nr;
-    for (int e = lane; e < nx; e += kCols) {
-      const int cc = e / nr;
-      const int q = e - cc * nr;
-      lhs[sbase[cc] + sind[r0 + q]] = sx[cc * PITCH_X + q];
-    }
-  }
-}
-
 // columnwise_op_appinv with LDS-staged loads (FP32 throughout): the bands
 // of a workgroup's 64 columns are one contiguous block (3 NROW values per
 // column), so each kCh-row stage is read by instructions covering a few
-// columns' contiguous runs (the per-lane loads of k_appinv touch 64 lines
+// columns' contiguous runs (one lane's loads of its own column touch 64 lines
 // per instruction), all of a stage's loads issued before its LDS writes; the
-// recurrence is k_appinv's term for term with c' and d' in registers.
+// recurrence is the reference's term for term with c' and d' in registers.
 template <typename T, int NROW>
 __global__ void __launch_bounds__(kCols)
 k_appinv_staged(T* __restrict__ lhs, const T* __restrict__ x, const T* __restrict__ cm,
@@ -244,8 +155,8 @@ k_appinv_staged(T* __restrict__ lhs, const T* __restrict__ x, const T* __restric
 // columns are contiguous).  The right-hand side goes to LDS, each band stage
 // goes to LDS before its rows are solved (odd pitches: conflict-free per-lane
 // reads), the solution goes back through LDS and out in the same flat order
-// with streaming stores.  The recurrence is k_appinv's term for term, so the
-// bits are the same.
+// with streaming stores.  The recurrence is the reference's term for term, so
+// the bits are the same.
 // DPL: d' lives in the column's right-hand-side slots in LDS (each row reads
 // its right-hand side once, then holds d'), so a lane keeps only c' in
 // registers (about 70 fewer VGPRs, more waves per SIMD) and the backward
@@ -396,8 +307,8 @@ k_appinv_deep(float* __restrict__ lhs, const float* __restrict__ x, const float*
   }
 }
 
-// FP32 appinv kernel choice: 1 the unpipelined staged kernel, 0 the per-lane
-// k_appinv (LFR_APPINV_STAGED=0/1); otherwise the up-front-load kernel.
+// FP32 appinv kernel choice at 70 rows: 1 the unpipelined staged kernel, 0
+// k_thomas_rows (LFR_APPINV_STAGED=0/1); otherwise the up-front-load kernel.
 int appinv_variant() {
   static const int v = [] {
     const char* e = getenv("LFR_APPINV_STAGED");
@@ -443,6 +354,280 @@ k_appinv_generic(T* __restrict__ lhs, const T* __restrict__ x, const T* __restri
     }
     lhs[base + ind0(ind, i, nrow)] = (T)dpc[i];
   }
+}
+
+// ---------------------------------------------------------------------------
+// Thomas solves of any row count (k_thomas_rows), shared by appinv,
+// tri_solve and operator_tri_solve.  A solve is one serial recurrence a
+// column, so what bounds it is memory latency times dependent loads unless
+// the loads run ahead: a wave owns kRowCols columns and takes them in stages
+// of kRowStage rows, 16 lanes reading 16 consecutive rows of one column
+// (4 columns an instruction).  Two stages are in flight in registers while
+// the stage before them is solved from LDS by one lane a column; c' and d'
+// stay in LDS (2 nrow values a column, so all columns of a C64 mesh are
+// resident at once in FP64), the backward sweep leaves the solution in d' and
+// all lanes store it.  A one-lane-a-column kernel waits for a row's loads in
+// every row.  Arithmetic per row as the reference kernels (products commute
+// exactly; row 0 has a = 0 and starts from c' = d' = 0, which leaves its
+// pivot and right-hand side unchanged).
+// Measured (input sets in turn, µs, one-lane-a-column kernel with its loads
+// in the recurrence -> this one): operator_tri_solve C64L85 FP64 333 -> 30,
+// C96L30 FP64 201 -> 23; appinv C64L85 FP32 140 -> 17.5, C80L100 FP64 363 ->
+// 49; against the unrolled kernels that a few row counts had before: appinv
+// C96L70 FP64 75.6 -> 45.5 (3.4 TB/s), C96L30 FP32 12.5 -> 11.7.  32 columns
+// a wave or 8 rows a stage were 5 to 40 % slower, 8 columns 3 to 45 %.
+// ---------------------------------------------------------------------------
+constexpr int kRowCols = 16;
+constexpr int kRowStage = 16;
+constexpr size_t kRowLdsMax = 64 * 1024;   // dynamic LDS of one workgroup
+
+// Sources of row r of a column: first the values that are addressed by cell
+// alone, then those that wait for the column's base (first dof) and the row's
+// dof offset; then (a, d, u, x) of the row from both.
+template <typename T>
+struct RowsBands {   // columnwise_matrix(3, nrow, ncell) and a field
+  static constexpr int kCell = 3, kField = 1;
+  const T* cm;
+  const T* x;
+  int nrow;
+  __device__ void load_cell(T* v, int c, int r) const {
+    const T* b = cm + ((int64_t)c * nrow + r) * 3;
+    v[0] = b[0];
+    v[1] = b[1];
+    v[2] = b[2];
+  }
+  __device__ void load_field(T* v, int64_t base, int off) const { v[0] = x[base + off]; }
+  __device__ void row(const T* vc, const T* vf, int r, T (&o)[4]) const {
+    o[0] = r ? vc[0] : T(0);
+    o[1] = vc[1];
+    o[2] = vc[2];
+    o[3] = vf[0];
+  }
+};
+
+template <typename T>
+struct RowsFields {   // tri_minus, tri_0, tri_plus, x
+  static constexpr int kCell = 0, kField = 4;
+  const T *tm, *t0, *tp, *x;
+  __device__ void load_cell(T*, int, int) const {}
+  __device__ void load_field(T* v, int64_t base, int off) const {
+    v[0] = tm[base + off];
+    v[1] = t0[base + off];
+    v[2] = tp[base + off];
+    v[3] = x[base + off];
+  }
+  __device__ void row(const T*, const T* vf, int r, T (&o)[4]) const {
+    o[0] = r ? vf[0] : T(0);
+    o[1] = vf[1];
+    o[2] = vf[2];
+    o[3] = vf[3];
+  }
+};
+
+template <typename T>
+struct RowsLma {   // 2x2 local matrices m(ik, i, j) at ik + n3 (i + 2 j), and x
+  static constexpr int kCell = 4, kField = 1;
+  const T *m, *x;
+  int nl;
+  int64_t n3;
+  __device__ void load_cell(T* v, int c, int r) const {
+    const int64_t ik = (int64_t)c * nl + r;
+    const int64_t ia = r < nl ? ik : ik - 1;   // layer r, clamped at the top
+    const int64_t ib = r >= 1 ? ik - 1 : ik;   // layer r - 1, clamped at the bottom
+    v[0] = m[ib + n3];
+    v[1] = m[ia];
+    v[2] = m[ib + 3 * n3];
+    v[3] = m[ia + 2 * n3];
+  }
+  __device__ void load_field(T* v, int64_t base, int off) const { v[0] = x[base + off]; }
+  __device__ void row(const T* vc, const T* vf, int r, T (&o)[4]) const {
+    o[0] = r ? vc[0] : T(0);
+    o[1] = r == 0 ? vc[1] + T(0) : (r < nl ? vc[1] + vc[2] : vc[2]);
+    o[2] = r < nl ? vc[3] : T(0);
+    o[3] = vf[0];
+  }
+};
+
+template <typename T, typename C>
+size_t rows_lds(int nrow) {
+  return (size_t)kRowCols * (nrow | 1) * 2 * sizeof(C) + (size_t)kRowCols * (2 * kRowStage + 1) * sizeof(T);
+}
+
+// IND: row r of a column is dof ind[r] - 1 of it (clamped into the column);
+// else row r is dof r
+template <typename T, typename C, typename S, bool IND>
+__global__ void __launch_bounds__(64)
+k_thomas_rows(T* __restrict__ y, S src, const int32_t* __restrict__ map0, int ndf, int cstride,
+              const int32_t* __restrict__ ind, int ncell, int nrow) {
+  constexpr int CI = 64 / kRowStage;           // columns an instruction covers
+  constexpr int G = kRowCols / CI;             // load slots a lane
+  constexpr int PB = 2 * kRowStage + 1;    // odd pitches: conflict-free per-lane access
+  extern __shared__ double smem_rows[];
+  const int PC = nrow | 1;
+  C* scp = reinterpret_cast<C*>(smem_rows);   // u, then c'
+  C* sdp = scp + kRowCols * PC;               // x, then d', then the solution
+  T* sb = reinterpret_cast<T*>(sdp + kRowCols * PC);   // a and d of the stage
+  const int lane = threadIdx.x;
+  const int rl = lane % kRowStage, g = lane / kRowStage;
+  const int c0 = blockIdx.x * kRowCols;
+  const int ncols = min(kRowCols, ncell - c0);
+  const int nst = (nrow + kRowStage - 1) / kRowStage;
+  // slot it of a lane: row rl of the stage, column 4 it + g; rows and columns
+  // past the end repeat the last (in bounds, never used)
+  int cell[G];
+  int64_t base[G];
+#pragma unroll
+  for (int it = 0; it < G; ++it) cell[it] = c0 + min(CI * it + g, ncols - 1);
+  if (cstride >= 0) {
+#pragma unroll
+    for (int it = 0; it < G; ++it) base[it] = cell[it] * cstride;
+  } else {
+    int32_t m[G];
+#pragma unroll
+    for (int it = 0; it < G; ++it) m[it] = map0[(int64_t)cell[it] * ndf];
+#pragma unroll
+    for (int it = 0; it < G; ++it) base[it] = m[it];
+  }
+  const auto row_of = [&](int s) { return min(s * kRowStage + rl, nrow - 1); };
+  // row offsets of a stage, raw: their loads go out a stage before the field
+  // loads that wait for them
+  const auto offset = [&](int s) { return IND ? ind[row_of(s)] : 0; };
+  const auto clamped = [&](int s, int o) { return IND ? min(max(o - 1, 0), nrow - 1) : row_of(s); };
+  struct Raw {
+    T c[G][S::kCell ? S::kCell : 1], f[G][S::kField];
+  } va, vb;
+  const auto fetch_cell = [&](int s, Raw& v) {
+    const int r = row_of(s);
+#pragma unroll
+    for (int it = 0; it < G; ++it) src.load_cell(v.c[it], cell[it], r);
+  };
+  const auto fetch_field = [&](Raw& v, int off) {
+#pragma unroll
+    for (int it = 0; it < G; ++it) src.load_field(v.f[it], base[it], off);
+  };
+  const int off0 = offset(0), off1 = offset(1);
+  int off = offset(2);
+  fetch_cell(0, va);
+  fetch_field(va, clamped(0, off0));
+  fetch_cell(1, vb);   // a single stage reads its last row again
+  fetch_field(vb, clamped(1, off1));
+  C cprev = C(0), dprev = C(0);
+  // NR rows from row i0 + q0: their values are read before the chain needs them
+  const auto rows = [&](int i0, int q0, auto nr) {
+    constexpr int NR = decltype(nr)::value;
+    C a[NR], d[NR], u[NR], x[NR];
+#pragma unroll
+    for (int q = 0; q < NR; ++q) {
+      a[q] = (C)sb[lane * PB + 2 * (q0 + q)];
+      d[q] = (C)sb[lane * PB + 2 * (q0 + q) + 1];
+      u[q] = scp[lane * PC + i0 + q0 + q];
+      x[q] = sdp[lane * PC + i0 + q0 + q];
+    }
+#pragma unroll
+    for (int q = 0; q < NR; ++q) {
+      const C ac = a[q] * cprev;
+      const C inv = C(1) / (d[q] - ac);
+      cprev = inv * u[q];
+      const C ad = a[q] * dprev;
+      dprev = inv * (x[q] - ad);
+      scp[lane * PC + i0 + q0 + q] = cprev;
+      sdp[lane * PC + i0 + q0 + q] = dprev;
+    }
+  };
+  const auto stage = [&](int s, Raw& v, auto more) {
+    const int i0 = s * kRowStage, r = row_of(s);
+    // rows past the end hold the last row's values and write them there
+#pragma unroll
+    for (int it = 0; it < G; ++it) {
+      const int c = CI * it + g;
+      T o[4];
+      src.row(v.c[it], v.f[it], r, o);
+      sb[c * PB + 2 * rl] = o[0];
+      sb[c * PB + 2 * rl + 1] = o[1];
+      scp[c * PC + r] = (C)o[2];
+      sdp[c * PC + r] = (C)o[3];
+    }
+    __syncthreads();
+    if constexpr (decltype(more)::value) {
+      // not behind a branch (a stage past the end reads the last row again):
+      // the next stage's wait would be for every load in flight
+      const int o = clamped(s + 2, off);
+      off = offset(s + 3);
+      fetch_cell(s + 2, v);
+      fetch_field(v, o);
+    }
+    if (lane < kRowCols) {
+      if (i0 + kRowStage <= nrow) {
+#pragma unroll
+        for (int q = 0; q < kRowStage; q += 8) rows(i0, q, std::integral_constant<int, 8>{});
+      } else {
+        const int nr = nrow - i0;
+        int q = 0;
+        if (nr & 8) rows(i0, 0, std::integral_constant<int, 8>{}), q = 8;
+        if (nr & 4) rows(i0, q, std::integral_constant<int, 4>{}), q += 4;
+        for (; q < nr; ++q) rows(i0, q, std::integral_constant<int, 1>{});
+      }
+    }
+    __syncthreads();
+  };
+  int s = 0;
+  for (; s + 2 < nst; s += 2) {
+    stage(s, va, std::true_type{});
+    stage(s + 1, vb, std::true_type{});
+  }
+  stage(s, va, std::false_type{});
+  if (s + 1 < nst) stage(s + 1, vb, std::false_type{});
+  // backward substitution, 8 rows' c' and d' read ahead of the chain
+  if (lane < kRowCols) {
+    C* cpl = scp + lane * PC;
+    C* dpl = sdp + lane * PC;
+    C dn = dprev;
+    int i = nrow - 2;
+    for (; i >= 7; i -= 8) {
+      C cv[8], dv[8];
+#pragma unroll
+      for (int q = 0; q < 8; ++q) {
+        cv[q] = cpl[i - q];
+        dv[q] = dpl[i - q];
+      }
+#pragma unroll
+      for (int q = 0; q < 8; ++q) {
+        const C cd = cv[q] * dn;
+        dn = dv[q] - cd;
+        dpl[i - q] = dn;
+      }
+    }
+    for (; i >= 0; --i) {
+      const C cd = cpl[i] * dn;
+      dn = dpl[i] - cd;
+      dpl[i] = dn;
+    }
+  }
+  __syncthreads();
+  for (s = 0; s < nst; ++s) {
+    const int r = s * kRowStage + rl;
+    const int o = clamped(s, offset(s));
+#pragma unroll
+    for (int it = 0; it < G; ++it) {
+      const int c = CI * it + g;
+      if (c < ncols && r < nrow) __builtin_nontemporal_store((T)sdp[c * PC + r], y + base[it] + o);
+    }
+  }
+}
+
+// Queue a solve; false when the columns are too tall for its LDS
+template <typename C, typename T, typename S>
+bool launch_rows(hipStream_t s, T* y, const S& src, const lfr_space* sp, const int32_t* ind, int ncell, int nrow) {
+  const size_t lds = rows_lds<T, C>(nrow);
+  if (lds > kRowLdsMax) return false;
+  const dim3 grid((unsigned)((ncell + kRowCols - 1) / kRowCols));
+  if (ind)
+    hipLaunchKernelGGL((k_thomas_rows<T, C, S, true>), grid, dim3(64), lds, s, y, src, sp->map0_d, sp->ndf,
+                       sp->col_stride, ind, ncell, nrow);
+  else
+    hipLaunchKernelGGL((k_thomas_rows<T, C, S, false>), grid, dim3(64), lds, s, y, src, sp->map0_d, sp->ndf,
+                       sp->col_stride, ind, ncell, nrow);
+  return true;
 }
 
 template <typename T, typename C>
@@ -511,23 +696,13 @@ int launch_appinv(lfr_ctx* ctx, T* lhs, const T* x, const T* cm, const lfr_space
       return LFR_OK;
     }
   }
-  switch (nrow) {
-#define CASE(NR)                                                                              \
-  case NR:                                                                                    \
-    hipLaunchKernelGGL((k_appinv<T, C, NR>), dim3(nb), dim3(kCols), 0, ctx->stream, lhs, x, cm, \
-                       sp->map0_d, sp->ndf, ind, ncell);                                      \
-    break;
-    CASE(3) CASE(4) CASE(10) CASE(11) CASE(20) CASE(21) CASE(30) CASE(31) CASE(50) CASE(51)
-    CASE(70) CASE(71)
-#undef CASE
-    default: {
-      // c', d' scratch for row counts without a compiled kernel
-      int rc = lfr_work_reserve(ctx, (size_t)ncell * 2 * nrow * sizeof(C) + 4096);
-      if (rc) return rc;
-      hipLaunchKernelGGL((k_appinv_generic<T, C>), dim3(nb), dim3(kCols), 0, ctx->stream, lhs, x,
-                         cm, sp->map0_d, sp->ndf, ind, ncell, nrow,
-                         (C*)((char*)ctx->work + 4096));
-    }
+  if (!launch_rows<C>(ctx->stream, lhs, RowsBands<T>{cm, x, nrow}, sp, ind, ncell, nrow)) {
+    // c', d' scratch for columns taller than k_thomas_rows holds
+    int rc = lfr_work_reserve(ctx, (size_t)ncell * 2 * nrow * sizeof(C) + 4096);
+    if (rc) return rc;
+    hipLaunchKernelGGL((k_appinv_generic<T, C>), dim3(nb), dim3(kCols), 0, ctx->stream, lhs, x,
+                       cm, sp->map0_d, sp->ndf, ind, ncell, nrow,
+                       (C*)((char*)ctx->work + 4096));
   }
   LFR_CHECK_LAUNCH(ctx);
   return LFR_OK;
@@ -1104,86 +1279,6 @@ k_operator_tri_solve(T* __restrict__ y, const T* __restrict__ x, const T* __rest
   }
 }
 
-// tri_solve in the form of k_appinv: one lane per column, 64 columns per
-// workgroup, the column's bands and right-hand side loaded straight from
-// global memory (each a constant offset from one per-lane base: the W3 dofs
-// of a column are contiguous) kPf rows ahead of the recurrence, c' in LDS
-// and d' in registers (NROW a compile-time constant), the solution stored
-// through LDS.  The arithmetic is k_tri_solve's term for term (products
-// commute exactly), so the bits are the same.
-template <typename T, int NROW>
-__global__ void __launch_bounds__(kCols)
-k_thomas(T* __restrict__ y, const T* __restrict__ x, const T* __restrict__ t0, const T* __restrict__ tp,
-         const T* __restrict__ tm, const int32_t* __restrict__ map0, int ndf, int ncell) {
-  constexpr int NST = (NROW + kCh - 1) / kCh;
-  constexpr int PITCH_X = kCh + 1;                 // odd pitch: conflict-free lane-strided access
-  __shared__ T sx[kCols * PITCH_X];
-  __shared__ int32_t sbase[kCols];
-  constexpr int PC = NROW | 1;     // odd pitch of the c' rows
-  __shared__ T scp[kCols * PC];    // c' of every lane's column (registers hold d')
-  const int lane = threadIdx.x;
-  const int c0 = blockIdx.x * kCols;
-  const int ncols = min(kCols, ncell - c0);
-  if (lane < ncols) sbase[lane] = map0[(int64_t)(c0 + lane) * ndf];
-  T* cp = scp + lane * PC;
-  T dp[NROW];
-  {
-    const int cl = min(lane, ncols - 1);   // idle lanes of a partial workgroup repeat a real column
-    const int64_t base = map0[(int64_t)(c0 + cl) * ndf];
-    T la[NROW], ld[NROW], lu[NROW], lx[NROW];
-#pragma unroll
-    for (int t = 0; t < NROW + kPf; ++t) {
-      if (t < NROW) {
-        la[t] = tm[base + t];
-        ld[t] = t0[base + t];
-        lu[t] = tp[base + t];
-        lx[t] = x[base + t];
-      }
-      if (t >= kPf) {
-        const int i = t - kPf;
-        const T a = la[i], dg = ld[i], u = lu[i], xv = lx[i];
-        if (i == 0) {
-          const T inv = T(1) / dg;
-          cp[i] = u * inv;
-          dp[i] = xv * inv;
-        } else {
-          const T ac = a * cp[i - 1];
-          const T inv = T(1) / (dg - ac);
-          const T ad = a * dp[i - 1];
-          if (i < NROW - 1) cp[i] = u * inv;
-          dp[i] = (xv - ad) * inv;
-        }
-      }
-      // loads of rows [r kPf, (r+1) kPf) share a scheduling region with the
-      // recurrence of the kPf rows before them
-      if ((t + 1) % kPf == 0) __builtin_amdgcn_sched_barrier(0);
-    }
-  }
-#pragma unroll
-  for (int i = NROW - 2; i >= 0; --i) {
-    const T cd = cp[i] * dp[i + 1];
-    dp[i] = dp[i] - cd;
-  }
-#pragma unroll
-  for (int s = 0; s < NST; ++s) {
-    const int r0 = s * kCh;
-    const int nr = (NROW - r0) < kCh ? (NROW - r0) : kCh;
-    __syncthreads();
-    if (lane < ncols) {
-#pragma unroll
-      for (int q = 0; q < kCh; ++q)
-        if (r0 + q < NROW) sx[lane * PITCH_X + q] = dp[r0 + q];
-    }
-    __syncthreads();
-    const int nx = ncols * nr;
-    for (int e = lane; e < nx; e += kCols) {
-      const int cc = e / nr;
-      const int q = e - cc * nr;
-      y[(int64_t)sbase[cc] + r0 + q] = sx[cc * PITCH_X + q];
-    }
-  }
-}
-
 // tri_solve, FP32, every load issued at entry (the scheme of
 // k_appinv_deep): a wave owns COLS columns, loads the KCH-row stages of
 // tri_minus, tri_0, tri_plus and x of all its columns into registers up
@@ -1316,8 +1411,7 @@ k_thomas_deep(float* __restrict__ y, const float* __restrict__ x, const float* _
 // duplicates and are never read), all of a stage's loads issued before any
 // of its LDS writes (52 µs at C96L70 FP32 against 59 µs with each load
 // followed by its write), the recurrence runs from LDS with c' and d' in
-// registers.  For these four strided planes this beats the per-lane
-// direct loads of k_thomas.  Same arithmetic as k_operator_tri_solve.
+// registers.  Same arithmetic as k_operator_tri_solve.
 template <typename T, int NROW, int KCH>
 __global__ void __launch_bounds__(kCols)
 k_optri_staged(T* __restrict__ y, const T* __restrict__ x, const T* __restrict__ m,
@@ -1570,8 +1664,8 @@ bool launch_thomas(lfr_ctx* ctx, hipStream_t s, T* y, const T* x, const T* b0, c
   const unsigned nb = (unsigned)((sp->ncell + kCols - 1) / kCols);
   if constexpr (MODE == 0) {   // tri_solve: b0 = tri_0, b1 = tri_plus, b2 = tri_minus
     if constexpr (sizeof(T) == 4) {
-      // every load at entry (LFR_TRI_DEEP=0 keeps k_thomas); result-identical
-      // variants (columns a wave x rows a stage, k_thomas) chosen by the
+      // every load at entry (LFR_TRI_DEEP=0 keeps k_thomas_rows); result-identical
+      // variants (columns a wave x rows a stage, k_thomas_rows) chosen by the
       // autotuner on the first call of a shape (y never aliases an input)
       static const bool deep = [] {
         const char* e = getenv("LFR_TRI_DEEP");
@@ -1602,8 +1696,7 @@ bool launch_thomas(lfr_ctx* ctx, hipStream_t s, T* y, const T* x, const T* b0, c
                                  x, b0, b1, b2, sp->map0_d, sp->ndf, ncell, sp->col_stride);
               break;
             default:
-              hipLaunchKernelGGL((k_thomas<T, 70>), dim3(nb), dim3(kCols), 0, s, y, x, b0, b1, b2, sp->map0_d,
-                                 sp->ndf, ncell);
+              launch_rows<T>(s, y, RowsFields<T>{b2, b0, b1, x}, sp, nullptr, ncell, 70);
           }
           return hipGetLastError() == hipSuccess ? LFR_OK : LFR_ERR_HIP;
         };
@@ -1615,18 +1708,11 @@ bool launch_thomas(lfr_ctx* ctx, hipStream_t s, T* y, const T* x, const T* b0, c
         return true;
       }
     }
-    switch (sp->nlayers) {
-#define CASE(NR)                                                                                          \
-  case NR:                                                                                                \
-    hipLaunchKernelGGL((k_thomas<T, NR>), dim3(nb), dim3(kCols), 0, s, y, x, b0, b1, b2, sp->map0_d, sp->ndf, \
-                       sp->ncell);                                                                        \
-    return true;
-      CASE(10) CASE(70)
-#undef CASE
-      default: return false;
-    }
+    return launch_rows<T>(s, y, RowsFields<T>{b2, b0, b1, x}, sp, nullptr, sp->ncell, sp->nlayers);
   } else {                     // operator_tri_solve: b0 = the 2x2 local matrices
-    if (sp->nlayers != 70) return false;
+    if (sp->nlayers != 70 || sizeof(T) == 8)
+      return launch_rows<T>(s, y, RowsLma<T>{b0, x, sp->nlayers, (int64_t)sp->ncell * sp->nlayers}, sp, nullptr,
+                            sp->ncell, sp->nlayers + 1);
     if constexpr (sizeof(T) == 4) {
       // result-identical variants (columns a wave x rows a stage, the staged
       // kernel) chosen by the autotuner on the first call of a shape
@@ -1656,9 +1742,7 @@ bool launch_thomas(lfr_ctx* ctx, hipStream_t s, T* y, const T* x, const T* b0, c
       (void)launch(c);
       return true;
     }
-    hipLaunchKernelGGL((k_optri_staged<T, 71, kCh>), dim3(nb), dim3(kCols), 0, s, y, x, b0, sp->map0_d,
-                       sp->ndf, sp->ncell, sp->nlayers);
-    return true;
+    return false;
   }
 }
 

@@ -86,3 +86,35 @@ def test_appinv_permuted_indirection(ctx, dtype, nc):
     api.columnwise_op_appinv(y, torch.from_numpy(x).to(ctx.device), op)
     torch.cuda.synchronize()
     np.testing.assert_array_equal(y.cpu().numpy(), ref)
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("nl", [1, 2, 7, 16, 17, 30, 32, 50, 85, 240])
+def test_appinv_any_height_bitexact(ctx, dtype, nl):
+    """Row counts around the 16-row stages, 54 columns (a partial wave), a
+    permuted indirection, lhs by itself and in place of x; FP64 pivots on FP32
+    data give the FP64 solve rounded to FP32 (the same operations in FP64)."""
+    from lfric_core_amd import api
+    print(f"case appinv C3 nl={nl} {dtype.__name__}", flush=True)
+    m = cubed_sphere(3)
+    w3 = build_dofmap(m, "W3", nl)
+    st = Stream(38)
+    cm = _helmholtz_columns(st, m.ncells, nl).astype(dtype)
+    x = st.uniform(w3.undf).astype(dtype)
+    ind = (np.random.default_rng(6).permutation(nl) + 1).astype(np.int32)
+    ref = oracle.appinv(np.zeros_like(x), x, cm, w3.dofmap, ind)
+    sp = api.Space(ctx, w3)
+    op = api.CMAOperator(torch.from_numpy(cm).to(ctx.device), sp, ind)
+    xd = torch.from_numpy(x).to(ctx.device)
+    y = torch.full((w3.undf,), float("nan"), dtype=op.matrix.dtype, device=ctx.device)
+    api.columnwise_op_appinv(y, xd, op)
+    z = xd.clone()
+    api.columnwise_op_appinv(z, z, op)
+    torch.cuda.synchronize()
+    np.testing.assert_array_equal(y.cpu().numpy(), ref)
+    np.testing.assert_array_equal(z.cpu().numpy(), ref)
+    if dtype == np.float32:
+        ref64 = oracle.appinv(np.zeros(w3.undf), x.astype(np.float64), cm.astype(np.float64), w3.dofmap, ind)
+        api.columnwise_op_appinv(y, xd, op, fp64_pivots=True)
+        torch.cuda.synchronize()
+        np.testing.assert_array_equal(y.cpu().numpy(), ref64.astype(np.float32))

@@ -122,3 +122,44 @@ def test_operator_tri_solve_columns_not_at_a_constant_stride(ctx):
     api.operator_tri_solve(y, _t(x, ctx), _t(m, ctx), sp)
     torch.cuda.synchronize()
     np.testing.assert_array_equal(y.cpu().numpy(), ref)
+
+
+# row counts around the 16-row stages of the solves (none, one and several
+# whole stages, every remainder form) and one too tall for their LDS in FP64
+ROWS = [1, 2, 7, 15, 16, 17, 31, 32, 33, 48, 61, 85, 240]
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("permuted", [False, True])
+@pytest.mark.parametrize("nl", ROWS)
+def test_tri_solves_of_any_height_bitexact(ctx, dtype, nl, permuted):
+    """54 columns (three waves of 16 and a partial one); permuted: the cells
+    point at a permutation of the column blocks, so bases come from the map."""
+    import dataclasses
+    from lfric_core_amd import api
+    print(f"case tri solves C3 nl={nl} permuted={permuted} {dtype.__name__}", flush=True)
+    mesh = cubed_sphere(3)
+    st = Stream(55)
+    for space in ("W3", "WTHETA"):
+        fs = build_dofmap(mesh, space, nl)
+        if permuted:
+            perm = np.random.default_rng(9).permutation(mesh.ncells)
+            fs = dataclasses.replace(fs, dofmap=np.ascontiguousarray(fs.dofmap[perm]))
+        sp = api.Space(ctx, fs)
+        x = st.uniform(fs.undf).astype(dtype)
+        y = torch.full((fs.undf,), float("nan"), dtype=torch.from_numpy(x).dtype, device=ctx.device)
+        if space == "W3":
+            t0 = (4.0 + st.uniform(fs.undf)).astype(dtype)
+            tp = (0.5 * st.uniform(fs.undf)).astype(dtype)
+            tm = (0.5 * st.uniform(fs.undf)).astype(dtype)
+            ref = oracle.tri_solve(np.zeros(fs.undf, dtype), x, t0, tp, tm, fs.dofmap, nl)
+            api.tri_solve(y, _t(x, ctx), _t(t0, ctx), _t(tp, ctx), _t(tm, ctx), sp)
+        else:
+            m = 0.5 * st.uniform(4 * mesh.ncells * nl).reshape(2, 2, -1)
+            m[0, 0] += 2.0
+            m[1, 1] += 2.0
+            m = m.astype(dtype)
+            ref = oracle.operator_tri_solve(np.zeros(fs.undf, dtype), x, m, fs.dofmap, nl)
+            api.operator_tri_solve(y, _t(x, ctx), _t(m, ctx), sp)
+        torch.cuda.synchronize()
+        np.testing.assert_array_equal(y.cpu().numpy(), ref)
