@@ -80,6 +80,10 @@ struct lfr_plan_class {
   int ncol = 0;
   int32_t* col_start_d = nullptr;   // (ncol) first dof of the column, 0-based
   int32_t* ent_d = nullptr;         // (ncol, ngroup*gsize, 2): cell (0-based), (i << 1) | shift
+  // bundles of bsize columns (1 or 4) with the same cells and shifts, for
+  // k_gather_bun (records: see there)
+  int nbund = 0, bsize = 1;
+  int32_t* bund_d = nullptr;
   std::vector<int32_t> starts_h;    // host copies, for compiling column records
   std::vector<int32_t> ent_h;
 };

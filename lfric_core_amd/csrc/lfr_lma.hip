@@ -136,12 +136,93 @@ void launch_gather_any(hipStream_t s, int kind, unsigned nb, const T* M, const T
     case 1: launch_gather_shape<T, 1>(s, kind, nb, M, x, y, mi, c, nl, n3, ndf_out, ndf_in, overwrite); break;
     case 6: launch_gather_shape<T, 6>(s, kind, nb, M, x, y, mi, c, nl, n3, ndf_out, ndf_in, overwrite); break;
     case 8: launch_gather_shape<T, 8>(s, kind, nb, M, x, y, mi, c, nl, n3, ndf_out, ndf_in, overwrite); break;
-    default:
-      if (c.gsize == 1)
-        launch_gather_t<T, 0, 0, 1>(s, kind, nb, M, x, y, mi, c, nl, n3, ndf_out, ndf_in, overwrite);
-      else
-        launch_gather_t<T, 0, 0, 2>(s, kind, nb, M, x, y, mi, c, nl, n3, ndf_out, ndf_in, overwrite);
+    default: break;   // run_bundles
   }
+}
+
+template <typename T, int F, bool QUAD>
+void launch_bundles(hipStream_t s, int kind, const T* M, const T* x, T* y, const int32_t* mi, const lfr::BunClasses& cl,
+                    int nl, int64_t n3, int ndf_out, int ndf_in, int nf, int overwrite) {
+  unsigned total = 0;
+  for (int c = 0; c < cl.n; ++c) total += cl.c[c].nblocks;
+  const unsigned nbp = pad8(total);
+  if (kind == 0)
+    hipLaunchKernelGGL((lfr::k_gather_bun<T, F, 0, QUAD>), dim3(nbp), dim3(kThreads), 0, s, M, x, y, mi, cl, total, nl,
+                       n3, ndf_out, ndf_in, nf, overwrite, nbp);
+  else
+    hipLaunchKernelGGL((lfr::k_gather_bun<T, F, 1, QUAD>), dim3(nbp), dim3(kThreads), 0, s, M, x, y, mi, cl, total, nl,
+                       n3, ndf_out, ndf_in, nf, overwrite, nbp);
+}
+
+template <typename T, int F>
+void launch_one(hipStream_t s, int kind, const T* M, const T* x, T* y, const int32_t* mi, const lfr::BunClass& bc,
+                int nl, int64_t n3, int ndf_out, int ndf_in, int nf, int overwrite) {
+  const unsigned nbp = pad8(bc.nblocks);
+#define LONE(GSV, KD, MK)                                                                                      \
+  hipLaunchKernelGGL((lfr::k_gather_one<T, F, GSV, KD, MK>), dim3(nbp), dim3(kThreads), 0, s, M, x, y, mi, bc, nl, n3, \
+                     ndf_out, ndf_in, nf, overwrite, nbp)
+  if (kind == 0) {
+    if (bc.gs == 0) LONE(1, 0, false); else if (bc.gs == 1) LONE(1, 0, true); else LONE(2, 0, true);
+  } else {
+    if (bc.gs == 0) LONE(1, 1, false); else if (bc.gs == 1) LONE(1, 1, true); else LONE(2, 1, true);
+  }
+#undef LONE
+}
+
+// Bundles of the first class a chunk of the interleaved launch takes (4 and
+// 64 measure the same)
+constexpr unsigned kBunChunk = 16;
+
+// nf fields ("ndata first") of a whole plan through the bundles of its
+// classes.  Fields per thread: with four rows a bundle and nf a multiple of 4,
+// the most that leave whole quads of lanes a level (k_gather_bun's quad form);
+// else 4, 2 or 1, the most that divide nf.
+template <typename T>
+int run_bundles(lfr_ctx* ctx, const lfr_plan* plan, int kind, const T* M, const T* x, T* y, const lfr_space* in,
+                int ndf_out, int64_t n3, int nf, int overwrite) {
+  const int nl = plan->space->nlayers;
+  hipStream_t s = ctx->stream;
+  const bool quad = nf % 4 == 0;
+  int F4 = nf % 2 == 0 ? 2 : 1;
+  if (quad)
+    for (F4 = 4; (nf / 4) % F4; --F4) {
+    }
+  const int F1 = nf % 4 == 0 ? 4 : (nf % 2 == 0 ? 2 : 1);
+  lfr::BunClasses cl = {};
+  const auto flush = [&]() {
+    if (!cl.n) return;
+    cl.nchunk = std::max(1u, (unsigned)cl.c[0].nbund / kBunChunk);
+#define LBF(FV, QV) launch_bundles<T, FV, QV>(s, kind, M, x, y, in->map0_d, cl, nl, n3, ndf_out, in->ndf, nf, overwrite)
+    if (quad) {
+      if (F4 == 4) LBF(4, true); else if (F4 == 3) LBF(3, true); else if (F4 == 2) LBF(2, true); else LBF(1, true);
+    } else {
+      if (F4 == 2) LBF(2, false); else LBF(1, false);
+    }
+#undef LBF
+    cl = {};
+  };
+  for (const auto& c : plan->classes) {
+    if (c.ncol == 0) continue;
+    LFR_REQUIRE(ctx, c.gsize == 1 || c.gsize == 2, "plan class with %d entries per cell unsupported", c.gsize);
+    lfr::BunClass b = {};
+    b.bund = c.bund_d;
+    b.nbund = c.nbund;
+    b.H = c.height;
+    b.ngroup = c.ngroup;
+    b.gs = c.gsize == 1 && c.height == nl ? 0 : c.gsize;
+    b.nblocks = lfr_blocks((int64_t)c.nbund * c.height * (nf / (c.bsize == 4 ? F4 : F1)), kThreads);
+    if (c.bsize == 4) {
+      if (cl.n == lfr::kBunMaxClass) flush();
+      cl.c[cl.n++] = b;
+    } else {
+#define LOF(FV) launch_one<T, FV>(s, kind, M, x, y, in->map0_d, b, nl, n3, ndf_out, in->ndf, nf, overwrite)
+      if (F1 == 4) LOF(4); else if (F1 == 2) LOF(2); else LOF(1);
+#undef LOF
+    }
+  }
+  flush();
+  LFR_CHECK_LAUNCH(ctx);
+  return LFR_OK;
 }
 
 template <typename T, int NDF_IN, int NG, int GS>
@@ -261,6 +342,8 @@ int run_gather(lfr_ctx* ctx, const lfr_plan* plan, int kind, const T* M, const T
     LFR_CHECK_LAUNCH(ctx);
     return LFR_OK;
   }
+  if (!pk && in->ndf != 1 && in->ndf != 6 && in->ndf != 8)
+    return run_bundles<T>(ctx, plan, kind, M, x, y, in, ndf_out, n3, 1, overwrite);
   for (size_t ci = 0; ci < plan->classes.size(); ++ci) {
     const auto& c = plan->classes[ci];
     if (c.ncol == 0) continue;
@@ -365,6 +448,52 @@ int check_pair(lfr_ctx* ctx, int prec, const void* lhs, const void* x, const voi
 // ---------------------------------------------------------------------------
 // Plan construction (host)
 // ---------------------------------------------------------------------------
+namespace {
+
+// Group a class's columns into bundles (lfr::k_gather_bun): runs of
+// consecutive columns whose entries name the same cells and shifts, up to
+// four a bundle; a class without such runs has one column a bundle.  Returns
+// the records and sets pc.nbund and pc.bsize.
+std::vector<int32_t> build_bundles(lfr_plan_class& pc) {
+  const int ne = pc.ngroup * pc.gsize, per = 2 * ne;
+  const auto alike = [&](int a, int b) {
+    const int32_t *ea = &pc.ent_h[(size_t)a * per], *eb = &pc.ent_h[(size_t)b * per];
+    for (int e = 0; e < ne; ++e) {
+      if (ea[2 * e] != eb[2 * e] || (ea[2 * e + 1] < 0) != (eb[2 * e + 1] < 0)) return false;
+      if (ea[2 * e + 1] >= 0 && ((ea[2 * e + 1] ^ eb[2 * e + 1]) & 1)) return false;
+    }
+    return true;
+  };
+  std::vector<std::pair<int, int>> runs;   // first column, count
+  for (int q = 0; q < pc.ncol; ++q) {
+    if (!runs.empty() && runs.back().second < 4 && alike(runs.back().first, q)) ++runs.back().second;
+    else runs.emplace_back(q, 1);
+  }
+  if (runs.size() * 2 > (size_t)pc.ncol) {   // under two columns a run: not worth the padding
+    runs.clear();
+    for (int q = 0; q < pc.ncol; ++q) runs.emplace_back(q, 1);
+    pc.bsize = 1;
+  } else {
+    pc.bsize = 4;
+  }
+  pc.nbund = (int)runs.size();
+  const int R = pc.bsize;
+  std::vector<int32_t> rec;
+  rec.reserve(runs.size() * (R + pc.ngroup * (1 + pc.gsize * R)));
+  for (const auto& run : runs) {
+    const auto col = [&](int r) { return run.first + std::min(r, run.second - 1); };
+    for (int r = 0; r < R; ++r) rec.push_back(pc.starts_h[col(r)]);
+    for (int g = 0; g < pc.ngroup; ++g) {
+      rec.push_back(pc.ent_h[(size_t)run.first * per + (size_t)g * pc.gsize * 2]);
+      for (int q = 0; q < pc.gsize; ++q)
+        for (int r = 0; r < R; ++r) rec.push_back(pc.ent_h[(size_t)col(r) * per + (size_t)(g * pc.gsize + q) * 2 + 1]);
+    }
+  }
+  return rec;
+}
+
+}  // namespace
+
 extern "C" int lfr_plan_create(lfr_ctx* ctx, const lfr_space* sp, const int32_t* cic,
                                const int32_t* npc, int ncolour, int maxc, int kind,
                                lfr_plan** out) {
@@ -495,18 +624,23 @@ extern "C" int lfr_plan_create(lfr_ctx* ctx, const lfr_space* sp, const int32_t*
     }
     pc.starts_h = starts;
     pc.ent_h = ent;
+    const std::vector<int32_t> bund = build_bundles(pc);
     const size_t b1 = starts.size() * sizeof(int32_t), b2 = ent.size() * sizeof(int32_t);
-    if (hipMalloc(&pc.col_start_d, b1) != hipSuccess || hipMalloc(&pc.ent_d, b2) != hipSuccess) {
+    const size_t b3 = bund.size() * sizeof(int32_t);
+    if (hipMalloc(&pc.col_start_d, b1) != hipSuccess || hipMalloc(&pc.ent_d, b2) != hipSuccess ||
+        hipMalloc(&pc.bund_d, b3) != hipSuccess) {
+      plan->classes.push_back(pc);
       lfr_plan_destroy(plan);
       return lfr_set_error(ctx, LFR_ERR_NOMEM, "plan allocation failed");
     }
     if (hipMemcpy(pc.col_start_d, starts.data(), b1, hipMemcpyHostToDevice) != hipSuccess ||
-        hipMemcpy(pc.ent_d, ent.data(), b2, hipMemcpyHostToDevice) != hipSuccess) {
+        hipMemcpy(pc.ent_d, ent.data(), b2, hipMemcpyHostToDevice) != hipSuccess ||
+        hipMemcpy(pc.bund_d, bund.data(), b3, hipMemcpyHostToDevice) != hipSuccess) {
       plan->classes.push_back(pc);
       lfr_plan_destroy(plan);
       return lfr_set_error(ctx, LFR_ERR_HIP, "plan upload failed");
     }
-    plan->nbytes += (int64_t)(b1 + b2);
+    plan->nbytes += (int64_t)(b1 + b2 + b3);
     plan->classes.push_back(pc);
   }
   *out = plan;
@@ -685,6 +819,7 @@ extern "C" int lfr_plan_destroy(lfr_plan* plan) {
   for (auto& c : plan->classes) {
     if (c.col_start_d) (void)hipFree(c.col_start_d);
     if (c.ent_d) (void)hipFree(c.ent_d);
+    if (c.bund_d) (void)hipFree(c.bund_d);
   }
   delete plan;
   return LFR_OK;
@@ -943,67 +1078,6 @@ extern "C" int lfr_matrix_vector_packed(lfr_ctx* ctx, const lfr_lma_packed* pk, 
 // ---------------------------------------------------------------------------
 // Multidata (ndata fields, "ndata first") apply
 // ---------------------------------------------------------------------------
-namespace {
-// fields per thread of the multidata gather: the widest of 16/8/4/1 that
-// divides ndata, capped at 4 (measured fastest on the 16-field FP64 W2
-// order-1 apply: 13.8 ms against 16.5 with 8 and 23.2 with 16);
-// LFR_NDATA_FPT=1/4/8/16 sets another cap
-int ndata_fpt(int nd) {
-  static const int cap = [] {
-    const char* e = getenv("LFR_NDATA_FPT");
-    const int v = e ? atoi(e) : 4;
-    return (v == 1 || v == 4 || v == 8 || v == 16) ? v : 4;
-  }();
-  for (int f : {16, 8, 4})
-    if (f <= cap && nd % f == 0) return f;
-  return 1;
-}
-
-template <typename T>
-int run_gather_ndata(lfr_ctx* ctx, const lfr_plan* plan, const T* M, const T* x, T* y, const lfr_space* in,
-                     int ndf_out, int64_t n3, int nd, int overwrite) {
-  const int nl = plan->space->nlayers;
-  for (const auto& c : plan->classes) {
-    if (c.ncol == 0) continue;
-    LFR_REQUIRE(ctx, c.gsize == 1 || c.gsize == 2, "plan class with %d entries per cell unsupported", c.gsize);
-    const int fpt = ndata_fpt(nd);
-    const unsigned nbp = pad8(lfr_blocks((int64_t)c.ncol * c.height * (nd / fpt), kThreads));
-#define LND(GSV, KD, F)                                                                                       \
-  hipLaunchKernelGGL((lfr::k_gather_nf<T, GSV, KD, F>), dim3(nbp), dim3(kThreads), 0, ctx->stream, M, x, y,  \
-                     in->map0_d, c.col_start_d, c.ent_d, c.ncol, c.height, c.ngroup, nl, n3, ndf_out, in->ndf, nd, \
-                     overwrite, nbp)
-    if (fpt == 16) {
-      if (plan->kind == 0) {
-        if (c.gsize == 1) LND(1, 0, 16); else LND(2, 0, 16);
-      } else {
-        if (c.gsize == 1) LND(1, 1, 16); else LND(2, 1, 16);
-      }
-    } else if (fpt == 8) {
-      if (plan->kind == 0) {
-        if (c.gsize == 1) LND(1, 0, 8); else LND(2, 0, 8);
-      } else {
-        if (c.gsize == 1) LND(1, 1, 8); else LND(2, 1, 8);
-      }
-    } else if (fpt == 4) {
-      if (plan->kind == 0) {
-        if (c.gsize == 1) LND(1, 0, 4); else LND(2, 0, 4);
-      } else {
-        if (c.gsize == 1) LND(1, 1, 4); else LND(2, 1, 4);
-      }
-    } else {
-      if (plan->kind == 0) {
-        if (c.gsize == 1) LND(1, 0, 1); else LND(2, 0, 1);
-      } else {
-        if (c.gsize == 1) LND(1, 1, 1); else LND(2, 1, 1);
-      }
-    }
-#undef LND
-    LFR_CHECK_LAUNCH(ctx);
-  }
-  return LFR_OK;
-}
-}  // namespace
-
 extern "C" int lfr_matrix_vector_ndata(lfr_ctx* ctx, int prec, void* lhs, const void* x, const void* M,
                                        const lfr_space* lhs_space, const lfr_space* x_space, const lfr_plan* plan,
                                        int ndata, int overwrite) {
@@ -1016,10 +1090,10 @@ extern "C" int lfr_matrix_vector_ndata(lfr_ctx* ctx, int prec, void* lhs, const 
               "lfr_matrix_vector_ndata: plan must be a plan of the output space");
   const int64_t n3 = (int64_t)lhs_space->ncell * lhs_space->nlayers;
   if (prec == 4)
-    return run_gather_ndata<float>(ctx, plan, (const float*)M, (const float*)x, (float*)lhs, x_space,
-                                   lhs_space->ndf, n3, ndata, overwrite);
-  return run_gather_ndata<double>(ctx, plan, (const double*)M, (const double*)x, (double*)lhs, x_space,
-                                  lhs_space->ndf, n3, ndata, overwrite);
+    return run_bundles<float>(ctx, plan, plan->kind, (const float*)M, (const float*)x, (float*)lhs, x_space,
+                              lhs_space->ndf, n3, ndata, overwrite);
+  return run_bundles<double>(ctx, plan, plan->kind, (const double*)M, (const double*)x, (double*)lhs, x_space,
+                             lhs_space->ndf, n3, ndata, overwrite);
 }
 
 static int dg_common(lfr_ctx* ctx, int prec, void* lhs, const void* x, const void* M,

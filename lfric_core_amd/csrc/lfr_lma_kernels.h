@@ -1,6 +1,8 @@
 // LMA apply kernels shared by the apply entry points and the fused solvers.
 #pragma once
 
+#include <type_traits>
+
 #include "lfr_internal.h"
 #include "lfr_reduce.h"
 
@@ -461,101 +463,451 @@ k_gather_vec(const T* __restrict__ M, const T* __restrict__ x, T* __restrict__ y
 }
 
 // ---------------------------------------------------------------------------
-// k_gather for nf fields at once (a multidata field, "ndata first": element
-// (dof d, field r) at d*nf + r).  Thread <-> (column, level, FPT fields); the
-// threads of one output dof sit side by side in a wavefront, so a matrix
-// element is one load shared by nf/FPT lanes and each operand dof is one
-// nf-wide contiguous read.  The terms of every field are added in exactly the
-// order of k_gather's runtime-ndf path (bit-identical to NF single-field
-// applies).
+// Gather of bundles: R output columns of one mesh entity (the dofs of an
+// order-1 face or cell interior) have the same cells and layer shifts, so they
+// read the same operand values; a thread takes R columns x F fields of one
+// level ("ndata first" fields: element (dof d, field r) at d*nf + r; nf = 1
+// is a single field).  A field value is then loaded once for R rows and a
+// matrix value once for F fields; with one row a thread, what bounded the
+// sixteen-field FP64 apply was not HBM but the operand traffic out of L1 (36
+// values x 16 fields for every row of 36 matrix values).  The nf / F threads
+// of one level sit side by side in a wavefront.  Record of a bundle (ints):
+//   [ g0[R] | per group: cell, per entry q: code[R] ]
+// (code = (local dof << 1) | shift, -1 for an absent entry; short bundles
+// repeat their last column and do not store it).  The terms of every field
+// are added in the order of k_gather (bit-identical results).
+// One launch takes all classes of a plan with four rows a bundle: their
+// blocks are interleaved chunk by chunk so that the blocks in flight belong to
+// the same few cells and find their operand in L2 (a launch a class reads the
+// operand from HBM once per class: 3316 against 2520 µs below).  The fields of
+// a level are read in 16-byte pieces that lie side by side across its lanes.
+// Measured, W2 order 1 (36 x 36), a row a thread -> this form: 16 fields FP64
+// C32L70 6060 -> 2520 µs, FP32 C24L33 1155 -> 332 µs, one field FP64 C32L70
+// 1290 -> 850-990 µs (4.7-5.5 TB/s), FP32 990 -> 520 µs.  What bounds the 16
+// fields now is L1 (two of three accesses are the operand and the rows'
+// matrix values) and the 8 wavefronts a CU that its registers leave; two
+// fields a thread (more wavefronts) took 2970 µs, streaming matrix loads
+// 2620, a whole dofmap vector per load 2650.
 // ---------------------------------------------------------------------------
-template <typename T, int GS, int KIND, int FPT>
-__global__ void __launch_bounds__(kThreads)
-k_gather_nf(const T* __restrict__ M, const T* __restrict__ x, T* __restrict__ y,
-            const int32_t* __restrict__ map_in, const int32_t* __restrict__ col_start,
-            const int32_t* __restrict__ ent, int ncol, int H, int ngroup, int nl, int64_t n3, int ndf_out,
-            int ndf_in, int nf, int overwrite, unsigned nb_pad) {
-  // FPT fields per thread (nf % FPT == 0): thread <-> (column, level, field group)
-  const unsigned lb = lfr_xcd_block(blockIdx.x, nb_pad);
-  const int ng = nf / FPT;
-  const int64_t t = (int64_t)lb * kThreads + threadIdx.x;
-  const bool valid = t < (int64_t)ncol * H * ng;
+struct BunClass {
+  const int32_t* bund;
+  int nbund, H, ngroup;
+  int gs;              // entries a cell; 0: one, and every level has it
+  unsigned nblocks;
+};
+constexpr int kBunMaxClass = 6;
+struct BunClasses {
+  BunClass c[kBunMaxClass];
+  int n;
+  unsigned nchunk;
+};
+
+template <typename T, int R, int F, int GS, int KIND, bool MASK>
+__device__ __forceinline__ void gather_bun_body(const T* __restrict__ M, const T* __restrict__ x, T* __restrict__ y,
+                                                const int32_t* __restrict__ map_in, const BunClass& bc, unsigned blk,
+                                                int nl, int64_t n3, int ndf_out, int ndf_in, int nf, int overwrite) {
+  constexpr int P = F * (int)sizeof(T) > 16 ? F * (int)sizeof(T) / 16 : 1;   // pieces of F fields
+  constexpr int PF = F / P;
+  const int ng = nf / F, ngroup = bc.ngroup, H = bc.H;
+  const int64_t t = (int64_t)blk * kThreads + threadIdx.x;
+  const bool valid = t < (int64_t)bc.nbund * H * ng;
   const int64_t tt = valid ? t : 0;
   const int64_t slot = tt / ng;
-  const int r0 = (int)(tt - slot * ng) * FPT;
-  const int col = (int)(slot / H);
-  const int L = (int)(slot - (int64_t)col * H);
-  const int32_t g0 = col_start[col];
-  T acc[FPT];
-  if (overwrite || !valid) {
+  const int r0 = (int)(tt - slot * ng) * PF;   // fields r0 + p * (nf / P) + [0, PF)
+  const int ps = nf / P;
+  const int b = (int)(slot / H);
+  const int L = (int)(slot - (int64_t)b * H);
+  const int32_t* rec = bc.bund + (int64_t)b * (R + ngroup * (1 + GS * R));
+  int g0[R];
 #pragma unroll
-    for (int f = 0; f < FPT; ++f) acc[f] = T(0);
-  } else {
-    const LVec<T, FPT> yv = ldvec<T, FPT, false>(y + (int64_t)(g0 + L) * nf + r0);
+  for (int r = 0; r < R; ++r) g0[r] = rec[r];
+  T acc[R][F];
 #pragma unroll
-    for (int f = 0; f < FPT; ++f) acc[f] = yv.v[f];
-  }
-  const int32_t* e = ent + (int64_t)col * ngroup * GS * 2;
+  for (int r = 0; r < R; ++r)
+#pragma unroll
+    for (int p = 0; p < P; ++p) {
+      if (overwrite || !valid) {
+#pragma unroll
+        for (int f = 0; f < PF; ++f) acc[r][p * PF + f] = T(0);
+      } else {
+        const LVec<T, PF> yv = ldvec<T, PF, false>(y + (int64_t)(g0[r] + L) * nf + r0 + p * ps);
+#pragma unroll
+        for (int f = 0; f < PF; ++f) acc[r][p * PF + f] = yv.v[f];
+      }
+    }
   for (int g = 0; g < ngroup; ++g) {
-    const int32_t* eg = e + g * GS * 2;
-    const int cc = eg[0];
-    int ii[GS], kk[GS];
+    const int32_t* e = rec + R + g * (1 + GS * R);
+    const int cc = e[0];
+    const int32_t* mi = map_in + (int64_t)cc * ndf_in;
+    const T* pm[GS][R];
+    const T* px[GS];
     bool ok[GS];
 #pragma unroll
     for (int q = 0; q < GS; ++q) {
-      const int code = eg[2 * q + 1];
-      const int k = L - (code & 1);
-      ok[q] = code >= 0 && k >= 0 && k < nl;
-      ii[q] = code >= 0 ? (code >> 1) : 0;
-      kk[q] = k < 0 ? 0 : (k >= nl ? nl - 1 : k);
+      const int c0 = e[1 + q * R];
+      const int k = L - (c0 & 1);
+      ok[q] = !MASK || (c0 >= 0 && k >= 0 && k < nl);
+      const int kk = k < 0 ? 0 : (k >= nl ? nl - 1 : k);   // clamped: always in bounds
+      px[q] = x + (int64_t)kk * nf + r0;
+#pragma unroll
+      for (int r = 0; r < R; ++r) {
+        const int code = e[1 + q * R + r];
+        const int64_t i = code >= 0 ? (code >> 1) : 0;
+        pm[q][r] = M + (int64_t)cc * nl + kk + n3 * (KIND == 0 ? i : i * ndf_in);
+      }
     }
-    const int32_t* mi = map_in + (int64_t)cc * ndf_in;
-    if (KIND == 0) {
-      for (int j = 0; j < ndf_in; ++j) {
-        const int xbj = mi[j];
+    const int64_t js = KIND == 0 ? n3 * ndf_out : n3;   // one input dof further
+    T dot[GS][R][F];
+    if (KIND == 1) {
+#pragma unroll
+      for (int q = 0; q < GS; ++q)
+#pragma unroll
+        for (int r = 0; r < R; ++r)
+#pragma unroll
+          for (int f = 0; f < F; ++f) dot[q][r][f] = T(0);
+    }
+    // input dofs j .. j + U - 1: all loads, then the products in order
+    const auto dofs = [&](int j, auto un) {
+      constexpr int U = decltype(un)::value;
+      T m[GS][R][U], xv[GS][U][F];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int64_t xb = (int64_t)mi[j + u] * nf;
 #pragma unroll
         for (int q = 0; q < GS; ++q) {
-          const int64_t ik = (int64_t)cc * nl + kk[q];
-          const T m = M[ik + n3 * ((int64_t)ii[q] + (int64_t)ndf_out * j)];
-          const LVec<T, FPT> xv = ldvec<T, FPT, false>(x + (int64_t)(xbj + kk[q]) * nf + r0);
 #pragma unroll
-          for (int f = 0; f < FPT; ++f) {
-            const T p = m * xv.v[f];
-            const T s = acc[f] + p;
-            acc[f] = ok[q] ? s : acc[f];
+          for (int p = 0; p < P; ++p) {
+            const LVec<T, PF> v = ldvec<T, PF, false>(px[q] + xb + p * ps);
+#pragma unroll
+            for (int f = 0; f < PF; ++f) xv[q][u][p * PF + f] = v.v[f];
           }
+#pragma unroll
+          for (int r = 0; r < R; ++r) m[q][r][u] = pm[q][r][js * (j + u)];
         }
       }
-    } else {
 #pragma unroll
-      for (int q = 0; q < GS; ++q) {
-        const int64_t ik = (int64_t)cc * nl + kk[q];
-        T dot[FPT];
+      for (int u = 0; u < U; ++u)
 #pragma unroll
-        for (int f = 0; f < FPT; ++f) dot[f] = T(0);
-        for (int j = 0; j < ndf_in; ++j) {
-          const T m = M[ik + n3 * ((int64_t)j + (int64_t)ndf_in * ii[q])];
-          const LVec<T, FPT> xv = ldvec<T, FPT, false>(x + (int64_t)(mi[j] + kk[q]) * nf + r0);
+        for (int q = 0; q < GS; ++q) {
+          if (KIND == 0) {
+            // df2 outer, df inner; an entry without a layer here adds nothing
+            if (ok[q]) {
 #pragma unroll
-          for (int f = 0; f < FPT; ++f) {
-            const T p = m * xv.v[f];
-            dot[f] = dot[f] + p;
+              for (int r = 0; r < R; ++r)
+#pragma unroll
+                for (int f = 0; f < F; ++f) {
+                  const T p = m[q][r][u] * xv[q][u][f];
+                  acc[r][f] = acc[r][f] + p;
+                }
+            }
+          } else {
+#pragma unroll
+            for (int r = 0; r < R; ++r)
+#pragma unroll
+              for (int f = 0; f < F; ++f) {
+                const T p = m[q][r][u] * xv[q][u][f];
+                dot[q][r][f] = dot[q][r][f] + p;
+              }
           }
         }
+    };
+    // loads in flight against registers: two input dofs at a time where two
+    // entries' rows of FP64 pairs would not leave two waves a SIMD
+    constexpr int U = GS * R > 4 ? 2 : 4;
+    int j = 0;
+    for (; j + U <= ndf_in; j += U) dofs(j, std::integral_constant<int, U>{});
+    for (; j < ndf_in; ++j) dofs(j, std::integral_constant<int, 1>{});
+    if (KIND == 1) {
 #pragma unroll
-        for (int f = 0; f < FPT; ++f) {
-          const T s = acc[f] + dot[f];
-          acc[f] = ok[q] ? s : acc[f];
+      for (int q = 0; q < GS; ++q)
+        if (ok[q]) {
+#pragma unroll
+          for (int r = 0; r < R; ++r)
+#pragma unroll
+            for (int f = 0; f < F; ++f) acc[r][f] = acc[r][f] + dot[q][r][f];
         }
-      }
     }
   }
   if (valid) {
-    LVec<T, FPT> o;
 #pragma unroll
-    for (int f = 0; f < FPT; ++f) o.v[f] = acc[f];
-    *reinterpret_cast<LVec<T, FPT>*>(y + (int64_t)(g0 + L) * nf + r0) = o;
+    for (int r = 0; r < R; ++r) {
+      if (r > 0 && g0[r] == g0[r - 1]) break;   // repeated column of a short bundle
+#pragma unroll
+      for (int p = 0; p < P; ++p) {
+        LVec<T, PF> o;
+#pragma unroll
+        for (int f = 0; f < PF; ++f) o.v[f] = acc[r][p * PF + f];
+        *reinterpret_cast<LVec<T, PF>*>(y + (int64_t)(g0[r] + L) * nf + r0 + p * ps) = o;
+      }
+    }
   }
+}
+
+// The same for four rows and ndata a multiple of 4: the four lanes of a quad
+// hold the fields of one level, so each loads the matrix values of one of the
+// four rows and the others take them by a quad broadcast.  One load
+// instruction then brings four rows' values and a lane keeps a quarter of
+// them, which leaves registers for a block of U input dofs in flight ahead of
+// the one being summed (across the cells of a column too).
+template <int I, typename T>
+__device__ __forceinline__ T quad_bcast(T v) {
+  constexpr int ctrl = I * 0x55;   // every lane of the quad reads lane I
+  if constexpr (sizeof(T) == 4) {
+    return __builtin_bit_cast(T, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), ctrl, 0xf, 0xf, true));
+  } else {
+    struct I2 {
+      int a, b;
+    };
+    I2 i = __builtin_bit_cast(I2, v);
+    i.a = __builtin_amdgcn_mov_dpp(i.a, ctrl, 0xf, 0xf, true);
+    i.b = __builtin_amdgcn_mov_dpp(i.b, ctrl, 0xf, 0xf, true);
+    return __builtin_bit_cast(T, i);
+  }
+}
+
+template <typename T, int F, int GS, int KIND, bool MASK>
+__device__ __forceinline__ void gather_quad_body(const T* __restrict__ M, const T* __restrict__ x, T* __restrict__ y,
+                                                 const int32_t* __restrict__ map_in, const BunClass& bc, unsigned blk,
+                                                 int nl, int64_t n3, int ndf_out, int ndf_in, int nf, int overwrite) {
+  constexpr int R = 4;
+  constexpr int U = GS == 2 ? 2 : 4;
+  constexpr int PF = F * (int)sizeof(T) <= 16 ? F : (F % 2 == 0 ? 2 : 1);   // fields side by side in a lane
+  constexpr int P = F / PF;
+  const int ng = nf / F, ngroup = bc.ngroup, H = bc.H;
+  const int64_t t = (int64_t)blk * kThreads + threadIdx.x;
+  const bool valid = t < (int64_t)bc.nbund * H * ng;   // the same for a whole quad
+  const int64_t tt = valid ? t : (int64_t)(threadIdx.x & 3);
+  const int64_t slot = tt / ng;
+  const int a = (int)(tt - slot * ng);
+  const int r0 = a * PF, ps = ng * PF;   // fields r0 + p ps + [0, PF)
+  const int b = (int)(slot / H);
+  const int L = (int)(slot - (int64_t)b * H);
+  const int32_t* rec = bc.bund + (int64_t)b * (R + ngroup * (1 + GS * R));
+  int g0[R];
+#pragma unroll
+  for (int r = 0; r < R; ++r) g0[r] = rec[r];
+  T acc[R][F];
+#pragma unroll
+  for (int r = 0; r < R; ++r)
+#pragma unroll
+    for (int p = 0; p < P; ++p) {
+      if (overwrite || !valid) {
+#pragma unroll
+        for (int f = 0; f < PF; ++f) acc[r][p * PF + f] = T(0);
+      } else {
+        const LVec<T, PF> yv = ldvec<T, PF, false>(y + (int64_t)(g0[r] + L) * nf + r0 + p * ps);
+#pragma unroll
+        for (int f = 0; f < PF; ++f) acc[r][p * PF + f] = yv.v[f];
+      }
+    }
+  T dot[GS][R][F];
+  const auto zero_dot = [&] {
+#pragma unroll
+    for (int q = 0; q < GS; ++q)
+#pragma unroll
+      for (int r = 0; r < R; ++r)
+#pragma unroll
+        for (int f = 0; f < F; ++f) dot[q][r][f] = T(0);
+  };
+  if (KIND == 1) zero_dot();
+  const int64_t js = KIND == 0 ? n3 * ndf_out : n3;   // one input dof further
+  // the load cursor: input dofs jl.. of group gl
+  int gl = 0, jl = 0;
+  const int32_t* mi;
+  const T *pm[GS], *px[GS];
+  const auto enter = [&] {
+    const int32_t* e = rec + R + gl * (1 + GS * R);
+    const int cc = e[0];
+    mi = map_in + (int64_t)cc * ndf_in;
+#pragma unroll
+    for (int q = 0; q < GS; ++q) {
+      const int code = e[1 + q * R + (threadIdx.x & 3)];
+      const int k = L - (code & 1);
+      const int kk = k < 0 ? 0 : (k >= nl ? nl - 1 : k);   // clamped: always in bounds
+      const int64_t i = code >= 0 ? (code >> 1) : 0;
+      px[q] = x + (int64_t)kk * nf + r0;
+      pm[q] = M + (int64_t)cc * nl + kk + n3 * (KIND == 0 ? i : i * ndf_in);
+    }
+  };
+  struct Block {
+    T m[GS][U], xv[GS][U][F];
+  };
+  const auto load = [&](Block& v) {
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int j = min(jl + u, ndf_in - 1);
+      const int64_t xb = (int64_t)mi[j] * nf;
+#pragma unroll
+      for (int q = 0; q < GS; ++q) {
+        v.m[q][u] = pm[q][js * j];
+#pragma unroll
+        for (int p = 0; p < P; ++p) {
+          const LVec<T, PF> w = ldvec<T, PF, false>(px[q] + xb + p * ps);
+#pragma unroll
+          for (int f = 0; f < PF; ++f) v.xv[q][u][p * PF + f] = w.v[f];
+        }
+      }
+    }
+    // past the last group the cursor stays on its last block (in bounds, unused)
+    jl += U;
+    if (jl >= ndf_in && gl + 1 < ngroup) {
+      ++gl;
+      jl = 0;
+      enter();
+    }
+  };
+  bool ok[GS];
+  const auto one = [&](const Block& v, int u) {
+#pragma unroll
+    for (int q = 0; q < GS; ++q) {
+      const T m[R] = {quad_bcast<0>(v.m[q][u]), quad_bcast<1>(v.m[q][u]), quad_bcast<2>(v.m[q][u]),
+                      quad_bcast<3>(v.m[q][u])};
+      if (KIND == 0) {
+        // df2 outer, df inner; an entry without a layer here adds nothing
+        if (ok[q]) {
+#pragma unroll
+          for (int r = 0; r < R; ++r)
+#pragma unroll
+            for (int f = 0; f < F; ++f) {
+              const T p = m[r] * v.xv[q][u][f];
+              acc[r][f] = acc[r][f] + p;
+            }
+        }
+      } else {
+#pragma unroll
+        for (int r = 0; r < R; ++r)
+#pragma unroll
+          for (int f = 0; f < F; ++f) {
+            const T p = m[r] * v.xv[q][u][f];
+            dot[q][r][f] = dot[q][r][f] + p;
+          }
+      }
+    }
+  };
+  // the sum cursor: input dofs j.. of group g
+  int g = 0, j = 0;
+  const auto mask = [&] {
+#pragma unroll
+    for (int q = 0; q < GS; ++q) {
+      const int c0 = rec[R + g * (1 + GS * R) + 1 + q * R];
+      const int k = L - (c0 & 1);
+      ok[q] = !MASK || (c0 >= 0 && k >= 0 && k < nl);
+    }
+  };
+  const auto sum = [&](const Block& v) {
+    if (j + U <= ndf_in) {
+#pragma unroll
+      for (int u = 0; u < U; ++u) one(v, u);
+    } else {
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+        if (j + u < ndf_in) one(v, u);
+    }
+    j += U;
+    if (j >= ndf_in) {
+      if (KIND == 1) {
+#pragma unroll
+        for (int q = 0; q < GS; ++q)
+          if (ok[q]) {
+#pragma unroll
+            for (int r = 0; r < R; ++r)
+#pragma unroll
+              for (int f = 0; f < F; ++f) acc[r][f] = acc[r][f] + dot[q][r][f];
+          }
+        zero_dot();
+      }
+      ++g;
+      j = 0;
+      if (MASK && g < ngroup) mask();
+    }
+  };
+  enter();
+  mask();
+  Block va, vb;
+  load(va);
+  const int nblk = ngroup * ((ndf_in + U - 1) / U);
+  int i = 0;
+  for (; i + 1 < nblk; i += 2) {
+    load(vb);
+    __builtin_amdgcn_sched_barrier(0);
+    sum(va);
+    load(va);
+    __builtin_amdgcn_sched_barrier(0);
+    sum(vb);
+  }
+  if (i < nblk) sum(va);
+  if (valid) {
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      if (r > 0 && g0[r] == g0[r - 1]) break;   // repeated column of a short bundle
+#pragma unroll
+      for (int p = 0; p < P; ++p) {
+        LVec<T, PF> o;
+#pragma unroll
+        for (int f = 0; f < PF; ++f) o.v[f] = acc[r][p * PF + f];
+        *reinterpret_cast<LVec<T, PF>*>(y + (int64_t)(g0[r] + L) * nf + r0 + p * ps) = o;
+      }
+    }
+  }
+}
+
+// First block of chunk k of a class with n blocks
+__host__ __device__ __forceinline__ unsigned bun_first(unsigned k, unsigned n, unsigned nchunk) {
+  return (unsigned)((uint64_t)k * n / nchunk);
+}
+
+// QUAD: R = 4 and nf / F a multiple of 4
+template <typename T, int F, int KIND, bool QUAD>
+__global__ void __launch_bounds__(kThreads, sizeof(T) == 8 && F + KIND >= 3 ? 2 : 3)
+k_gather_bun(const T* __restrict__ M, const T* __restrict__ x, T* __restrict__ y, const int32_t* __restrict__ map_in,
+             BunClasses cl, unsigned total, int nl, int64_t n3, int ndf_out, int ndf_in, int nf, int overwrite,
+             unsigned nb_pad) {
+  const unsigned lb = lfr_xcd_block(blockIdx.x, nb_pad);
+  if (lb >= total) return;
+  // the chunk that holds block lb (chunks are class by class within), then
+  // the class and its block
+  const auto start = [&](unsigned k) {
+    unsigned s = 0;
+    for (int c = 0; c < cl.n; ++c) s += bun_first(k, cl.c[c].nblocks, cl.nchunk);
+    return s;
+  };
+  unsigned k = (unsigned)((uint64_t)lb * cl.nchunk / total);
+  while (k > 0 && start(k) > lb) --k;
+  while (k + 1 < cl.nchunk && start(k + 1) <= lb) ++k;
+  unsigned rest = lb - start(k);
+  for (int c = 0; c < cl.n; ++c) {
+    const unsigned f = bun_first(k, cl.c[c].nblocks, cl.nchunk);
+    const unsigned m = bun_first(k + 1, cl.c[c].nblocks, cl.nchunk) - f;
+    if (rest < m) {
+      const BunClass& bc = cl.c[c];
+      if constexpr (QUAD) {
+        if (bc.gs == 0)
+          gather_quad_body<T, F, 1, KIND, false>(M, x, y, map_in, bc, f + rest, nl, n3, ndf_out, ndf_in, nf, overwrite);
+        else if (bc.gs == 1)
+          gather_quad_body<T, F, 1, KIND, true>(M, x, y, map_in, bc, f + rest, nl, n3, ndf_out, ndf_in, nf, overwrite);
+        else
+          gather_quad_body<T, F, 2, KIND, true>(M, x, y, map_in, bc, f + rest, nl, n3, ndf_out, ndf_in, nf, overwrite);
+      } else {
+        if (bc.gs == 0)
+          gather_bun_body<T, 4, F, 1, KIND, false>(M, x, y, map_in, bc, f + rest, nl, n3, ndf_out, ndf_in, nf, overwrite);
+        else if (bc.gs == 1)
+          gather_bun_body<T, 4, F, 1, KIND, true>(M, x, y, map_in, bc, f + rest, nl, n3, ndf_out, ndf_in, nf, overwrite);
+        else
+          gather_bun_body<T, 4, F, 2, KIND, true>(M, x, y, map_in, bc, f + rest, nl, n3, ndf_out, ndf_in, nf, overwrite);
+      }
+      return;
+    }
+    rest -= m;
+  }
+}
+
+// One class with one column a bundle (no rows to share an operand value)
+template <typename T, int F, int GS, int KIND, bool MASK>
+__global__ void __launch_bounds__(kThreads)
+k_gather_one(const T* __restrict__ M, const T* __restrict__ x, T* __restrict__ y, const int32_t* __restrict__ map_in,
+             BunClass bc, int nl, int64_t n3, int ndf_out, int ndf_in, int nf, int overwrite, unsigned nb_pad) {
+  gather_bun_body<T, 1, F, GS, KIND, MASK>(M, x, y, map_in, bc, lfr_xcd_block(blockIdx.x, nb_pad), nl, n3, ndf_out,
+                                           ndf_in, nf, overwrite);
 }
 
 // ---------------------------------------------------------------------------

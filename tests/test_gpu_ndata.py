@@ -87,3 +87,43 @@ def test_ndata_bad_args(ctx):
     with pytest.raises(LfrError):   # different ndata
         api.matrix_vector_ndata(torch.zeros(u, 4, dtype=torch.float64, device=ctx.device),
                                 torch.zeros(u, 3, dtype=torch.float64, device=ctx.device), op)
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("space,k", [("W2", 1), ("W0", 1), ("W2", 2)])
+@pytest.mark.parametrize("nl", [1, 2, 5])
+def test_bundled_applies_bitexact(ctx, dtype, space, k, nl):
+    """Higher-order spaces, whose columns go four dofs of one mesh entity to a
+    thread (W2) or one (W0, 27 dofs a cell), against the oracle: one field,
+    and 1 to 20 fields (quads of lanes at multiples of 4, 4 to 1 fields a
+    thread), matrix_vector and its transpose, increment and overwrite."""
+    from lfric_core_amd import api
+    nc = 2 if k == 2 else 3
+    m, col, fs, sp = _setup(ctx, nc, nl, k, {space})
+    fs, sp = fs[space], sp[space]
+    st = Stream(33)
+    M = normal_lma(st, m.ncells * nl, fs.ndf, fs.ndf).astype(dtype)
+    op = api.LMAOperator(_t(M, ctx), sp, sp, col)
+    for nd in (1, 2, 3, 4, 8, 12, 16, 20):
+        print(f"case bundles {space} k={k} C{nc} nl={nl} nd={nd} {dtype.__name__}", flush=True)
+        X = st.uniform(fs.undf * nd).reshape(fs.undf, nd).astype(dtype)
+        Y0 = st.uniform(fs.undf * nd).reshape(fs.undf, nd).astype(dtype)
+        for kind in (0, 1):
+            yi = _t(Y0, ctx)
+            yo = torch.full_like(yi, float("nan"))
+            api.matrix_vector_ndata(yi, _t(X, ctx), op, transpose=kind == 1)
+            api.matrix_vector_ndata(yo, _t(X, ctx), op, overwrite=True, transpose=kind == 1)
+            torch.cuda.synchronize()
+            yi, yo = yi.cpu().numpy(), yo.cpu().numpy()
+            for r in sorted({0, nd // 2, nd - 1}):
+                xr, y0 = np.ascontiguousarray(X[:, r]), np.ascontiguousarray(Y0[:, r])
+                ref = oracle.invoke_coloured(kind, col, nl, y0.copy(), xr, M, fs.dofmap, fs.dofmap)
+                np.testing.assert_array_equal(yi[:, r], ref)
+                ref = oracle.invoke_coloured(kind, col, nl, np.zeros_like(y0), xr, M, fs.dofmap, fs.dofmap)
+                np.testing.assert_array_equal(yo[:, r], ref)
+                if nd == 1:
+                    single = api.matrix_vector if kind == 0 else api.transpose_matrix_vector
+                    ys = torch.empty(fs.undf, dtype=op.matrix.dtype, device=ctx.device)
+                    single(ys, _t(xr, ctx), op, overwrite=True)
+                    torch.cuda.synchronize()
+                    np.testing.assert_array_equal(ys.cpu().numpy(), ref)
