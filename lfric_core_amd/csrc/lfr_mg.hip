@@ -26,8 +26,7 @@
 // (cp_k and 1/(d_k + 4 sigma - a_k cp_{k-1})) depend only on the operator and
 // are computed once per level at set-up with the same operations the
 // recurrence would use, so results are bitwise those of the textbook sweep.
-// The forward sweep stores d'_k in the output field and the backward sweep
-// finishes it in place, so a thread holds no per-layer arrays.
+// d' waits for the backward sweep in registers (70 layers) or LDS.
 //
 // One V-cycle over all right-hand sides is captured into a hipGraph on first
 // use and replayed; each level's kernels use the workgroup size chosen by a
@@ -116,45 +115,6 @@ __global__ void k_mg_factor(T* __restrict__ cp, T* __restrict__ iv, const T* __r
     iv[ik] = inv;
     cprev = inv * bu[ik];
     cp[ik] = cprev;
-  }
-}
-
-// One damped line-Jacobi sweep: xo = xi + omega * D^{-1} (b - A xi); thread = (cell, rhs)
-template <typename T>
-__global__ void __launch_bounds__(256) k_mg_smooth(T* __restrict__ xo, const T* __restrict__ xi, const T* __restrict__ b,
-                                                   const T* __restrict__ ba, const T* __restrict__ bd,
-                                                   const T* __restrict__ bu, const T* __restrict__ cp,
-                                                   const T* __restrict__ iv, const int32_t* __restrict__ nb,
-                                                   int ncell, int nl, int lgR, T sigma, T omega) {
-  const int R = 1 << lgR;
-  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= (int64_t)ncell * R) return;
-  const int c = (int)(t >> lgR), r = (int)(t & (R - 1));
-  const int64_t plane = (int64_t)ncell * R;
-  T xm = 0, x0 = xi[t], dprev = 0;
-  for (int k = 0; k < nl; ++k) {
-    const int64_t i = (int64_t)k * plane + t;
-    const int64_t ik = (int64_t)k * ncell + c;
-    const T xp = (k + 1 < nl) ? xi[i + plane] : T(0);
-    const T ak = ba[ik], dk = bd[ik], uk = bu[ik];
-    T ax = ak * xm;
-    ax = ax + dk * x0;
-    ax = ax + uk * xp;
-    ax = ax + horiz(xi + (int64_t)k * plane, nb, c, R, r, x0, sigma);
-    const T res = b[i] - ax;
-    const T dp = k == 0 ? iv[ik] * res : iv[ik] * (res - ak * dprev);
-    xo[i] = dp;
-    dprev = dp;
-    xm = x0;
-    x0 = xp;
-  }
-  T dnext = 0;
-  for (int k = nl - 1; k >= 0; --k) {
-    const int64_t i = (int64_t)k * plane + t;
-    T dp = xo[i];
-    if (k < nl - 1) dp = dp - cp[(int64_t)k * ncell + c] * dnext;
-    xo[i] = xi[i] + omega * dp;
-    dnext = dp;
   }
 }
 
@@ -403,57 +363,85 @@ __global__ void __launch_bounds__(256) k_mg_resnorm_final(const double* __restri
   }
 }
 
-// LFRic W3 fields (field r at r*undf, dof = c*nl + k) -> [k][c][r], a tile of
-// TC cells per block staged through LDS (contiguous reads and writes).
+// LFRic W3 fields (field r at r*undf, dof = c*nl + k) <-> [k][c][r] through an
+// LDS tile of kCvPairs (cell, right-hand side) pairs: on one side a workgroup's
+// cells are one contiguous run a field, read (written) 16 bytes a lane, on the
+// other a layer's pairs are 256 contiguous bytes; neither side divides.  Reading
+// each column straight from memory, 16 bytes a lane at a time, refetched its
+// lines (64 columns a wave overrun L1).  C96L70, 8 fields FP32 (248 MB moved):
+// 125 µs to the layer-major layout and 108 back with a division per element,
+// 56 and 44 here; a whole solve of one V-cycle 1101 µs, 1017 with each column
+// straight from memory, 921 here.
 template <typename T>
-__global__ void __launch_bounds__(256) k_to_mg(T* __restrict__ out, const T* __restrict__ in, int ncell, int nl,
-                                               int R, int TC) {
-  extern __shared__ char smem_raw[];
-  T* tile = (T*)smem_raw;          // [R][TC*nl]
-  const int c0 = blockIdx.x * TC;
-  const int tc = min(TC, ncell - c0);
-  const int64_t undf = (int64_t)ncell * nl;
-  const int span = tc * nl;
-  for (int idx = threadIdx.x; idx < R * span; idx += blockDim.x) {
-    const int r = idx / span, j = idx - r * span;
-    tile[r * TC * nl + j] = in[(int64_t)r * undf + (int64_t)c0 * nl + j];
-  }
-  __syncthreads();
-  for (int idx = threadIdx.x; idx < R * span; idx += blockDim.x) {
-    const int r = idx % R, rest = idx / R;
-    const int cc = rest % tc, k = rest / tc;
-    out[((int64_t)k * ncell + c0 + cc) * R + r] = tile[r * TC * nl + cc * nl + k];
+constexpr int kCvPairs = 256 / (int)sizeof(T);
+
+template <typename T>
+size_t convert_lds(int nl, int R) {   // R runs of odd pitch
+  return (size_t)R * (((kCvPairs<T> / R) * nl) | 1) * sizeof(T);
+}
+
+template <typename T, bool TO>
+__global__ void __launch_bounds__(256) k_mg_convert(T* __restrict__ out, const T* __restrict__ in, int ncell, int nl,
+                                                    int lgR) {
+  constexpr int V = 16 / (int)sizeof(T), NP = kCvPairs<T>;
+  struct __attribute__((aligned(4))) Vec {   // runs start anywhere
+    T v[V];
+  };
+  extern __shared__ double smem_cv[];
+  T* tile = reinterpret_cast<T*>(smem_cv);
+  const int R = 1 << lgR, cells = NP >> lgR;
+  const int c0 = blockIdx.x * cells;
+  const int span = min(cells, ncell - c0) * nl, pitch = (cells * nl) | 1;
+  const int64_t n = (int64_t)ncell << lgR;
+  // the field side: a wave takes every fourth right-hand side's run
+  const auto field = [&] {
+    for (int r = threadIdx.x >> 6; r < R; r += 4) {
+      const int64_t base = ((int64_t)r * ncell + c0) * nl;
+      T* row = tile + r * pitch;
+      int j = (threadIdx.x & 63) * V;
+      for (; j + V <= span; j += 64 * V) {
+        Vec v;
+        if (TO) {
+          v = *reinterpret_cast<const Vec*>(in + base + j);
+#pragma unroll
+          for (int i = 0; i < V; ++i) row[j + i] = v.v[i];
+        } else {
+#pragma unroll
+          for (int i = 0; i < V; ++i) v.v[i] = row[j + i];
+          *reinterpret_cast<Vec*>(out + base + j) = v;
+        }
+      }
+      for (int i = 0; i < V && j + i < span; ++i) {   // the run's last, partial piece
+        if (TO) row[j + i] = in[base + j + i];
+        else out[base + j + i] = row[j + i];
+      }
+    }
+  };
+  const int p = threadIdx.x % NP;
+  const int64_t t = (int64_t)blockIdx.x * NP + p;
+  T* cell = tile + (p & (R - 1)) * pitch + (p >> lgR) * nl;
+  if (TO) {
+    field();
+    __syncthreads();
+    if (t < n)
+      for (int k = threadIdx.x / NP; k < nl; k += 256 / NP) out[(int64_t)k * n + t] = cell[k];
+  } else {
+    if (t < n) {
+#pragma unroll 8
+      for (int k = threadIdx.x / NP; k < nl; k += 256 / NP) cell[k] = in[(int64_t)k * n + t];
+    }
+    __syncthreads();
+    field();
   }
 }
 
-template <typename T>
-__global__ void __launch_bounds__(256) k_from_mg(T* __restrict__ out, const T* __restrict__ in, int ncell, int nl,
-                                                 int R, int TC) {
-  extern __shared__ char smem_raw[];
-  T* tile = (T*)smem_raw;
-  const int c0 = blockIdx.x * TC;
-  const int tc = min(TC, ncell - c0);
-  const int64_t undf = (int64_t)ncell * nl;
-  const int span = tc * nl;
-  for (int idx = threadIdx.x; idx < R * span; idx += blockDim.x) {
-    const int r = idx % R, rest = idx / R;
-    const int cc = rest % tc, k = rest / tc;
-    tile[r * TC * nl + cc * nl + k] = in[((int64_t)k * ncell + c0 + cc) * R + r];
-  }
-  __syncthreads();
-  for (int idx = threadIdx.x; idx < R * span; idx += blockDim.x) {
-    const int r = idx / span, j = idx - r * span;
-    out[(int64_t)r * undf + (int64_t)c0 * nl + j] = tile[r * TC * nl + j];
-  }
-}
-
-// The same sweep for a compile-time layer count: the layers are unrolled,
+// One damped line-Jacobi sweep, xo = xi + omega * D^{-1} (b - A xi), for a
+// compile-time layer count: the layers are unrolled,
 // every load (x of the layer, its four neighbours, b, the bands and the
 // Thomas factor) is issued PF layers ahead of the recurrence (scheduling
 // region g holds the loads of layers [g PF, (g+1) PF) and the sweep of the PF
-// layers before them), and d' stays in registers, so xo is written once
-// instead of written, re-read and rewritten.  Same operations in the same
-// order as k_mg_smooth.
+// layers before them), and d' stays in registers, so xo is written once.
+// Thread = (cell, rhs).
 template <typename T, int NL, int PF = 4, bool KX = false>
 __global__ void __launch_bounds__(256) k_mg_smooth_nl(T* __restrict__ xo, const T* __restrict__ xi,
                                                       const T* __restrict__ b, const Band4<T>* __restrict__ adui,
@@ -540,6 +528,142 @@ __global__ void __launch_bounds__(256) k_mg_smooth_nl(T* __restrict__ xo, const 
   }
 }
 
+// The same sweep for any layer count: layers in chunks of CH, a chunk's loads
+// (x one layer up, b, the four neighbours, the bands) in flight while the
+// chunk before it is summed, d' in LDS ([layer][lane], so xo is written once),
+// the backward sweep's cp a chunk of CB layers ahead.  KX keeps x in LDS too
+// instead of reading it again in the backward sweep.  One wave a workgroup: the
+// LDS of the columns, not registers, sets how many are in flight (8 waves a CU
+// at 70 layers FP32), and the chunks in flight make up for it.  Same operations
+// and order as k_mg_smooth_nl.  Against a sweep that loaded layer by layer and
+// kept d' in xo (one solve of one V-cycle, conversions as now): C96L60 FP32
+// 1790 -> 970 µs, C72L85 FP64 2870 -> 1821, C48L33 FP32 350 -> 164, C40L100
+// FP64 one field 1810 -> 800.  At 70 layers k_mg_smooth_nl stays: C96L70 FP32
+// 1018 against 1212 µs, FP64 2372 against 2555 (its registers hold twice the
+// columns that LDS does).
+template <typename T, bool KX>
+__global__ void __launch_bounds__(64) k_mg_smooth_rt(T* __restrict__ xo, const T* __restrict__ xi,
+                                                     const T* __restrict__ b, const Band4<T>* __restrict__ adui,
+                                                     const T* __restrict__ cp, const int32_t* __restrict__ nb,
+                                                     int ncell, int nl, int lgR, T sigma, T omega, unsigned nb_pad) {
+  constexpr int CH = 4, CB = 8;
+  extern __shared__ double smem_mg[];
+  T* sd = reinterpret_cast<T*>(smem_mg) + threadIdx.x;
+  T* sx = sd + nl * 64;   // KX only
+  const int R = 1 << lgR;
+  const int64_t t0 = (int64_t)lfr_xcd_block(blockIdx.x, nb_pad) * 64 + threadIdx.x;
+  const int64_t plane = (int64_t)ncell * R;
+  if (t0 >= plane) return;   // no barrier below: a lane uses its own LDS column only
+  const int64_t t = t0;
+  const int c = (int)(t >> lgR), r = (int)(t & (R - 1));
+  const int64_t o0 = (int64_t)nb[4 * c + 0] * R + r, o1 = (int64_t)nb[4 * c + 1] * R + r;
+  const int64_t o2 = (int64_t)nb[4 * c + 2] * R + r, o3 = (int64_t)nb[4 * c + 3] * R + r;
+  struct Chunk {
+    T xp[CH], b[CH], h[4][CH];
+    Band4<T> bv[CH];
+  };
+  // layers past the top read the top layer (in bounds, unused)
+  const auto load = [&](Chunk& v, int k0) {
+#pragma unroll
+    for (int u = 0; u < CH; ++u) {
+      const int k = min(k0 + u, nl - 1);
+      const T* xk = xi + (int64_t)k * plane;
+      v.xp[u] = xi[(int64_t)min(k + 1, nl - 1) * plane + t];
+      v.b[u] = b[(int64_t)k * plane + t];
+      v.bv[u] = adui[(int64_t)k * ncell + c];
+      v.h[0][u] = xk[o0];
+      v.h[1][u] = xk[o1];
+      v.h[2][u] = xk[o2];
+      v.h[3][u] = xk[o3];
+    }
+  };
+  T xm = T(0), x0 = xi[t], dprev = T(0);
+  const auto layer = [&](const Chunk& v, int u, int k) {
+    const T xp = k + 1 < nl ? v.xp[u] : T(0);
+    const Band4<T> bv = v.bv[u];
+    T ax = bv.a * xm;
+    ax = ax + bv.d * x0;
+    ax = ax + bv.u * xp;
+    const T s4 = v.h[0][u] + v.h[1][u];
+    const T s5 = s4 + v.h[2][u];
+    const T sn = s5 + v.h[3][u];
+    const T four = (T)4 * x0;
+    ax = ax + sigma * (four - sn);
+    const T res = v.b[u] - ax;
+    const T d = k == 0 ? bv.iv * res : bv.iv * (res - bv.a * dprev);
+    sd[k * 64] = d;
+    if (KX) sx[k * 64] = x0;
+    dprev = d;
+    xm = x0;
+    x0 = xp;
+  };
+  const auto chunk = [&](const Chunk& v, int k0) {
+    if (k0 + CH <= nl) {
+#pragma unroll
+      for (int u = 0; u < CH; ++u) layer(v, u, k0 + u);
+    } else {
+#pragma unroll
+      for (int u = 0; u < CH; ++u)
+        if (k0 + u < nl) layer(v, u, k0 + u);
+    }
+  };
+  Chunk va, vb;
+  load(va, 0);
+  load(vb, CH);
+  int k = 0;
+  for (; k + CH < nl; k += 2 * CH) {
+    chunk(va, k);
+    load(va, k + 2 * CH);
+    __builtin_amdgcn_sched_barrier(0);
+    chunk(vb, k + CH);
+    load(vb, k + 3 * CH);
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  if (k < nl) chunk(va, k);
+  // backward sweep, chunks of layers k, k - 1, ..., k - CB + 1
+  struct Back {
+    T cp[CB], x[CB];
+  };
+  const auto bload = [&](Back& v, int kt) {
+#pragma unroll
+    for (int u = 0; u < CB; ++u) {
+      const int q = max(kt - u, 0);
+      v.cp[u] = cp[(int64_t)q * ncell + c];
+      if (!KX) v.x[u] = xi[(int64_t)q * plane + t];
+    }
+  };
+  T dnext = T(0);
+  const auto bchunk = [&](const Back& v, int kt) {
+    T d[CB], xv[CB];
+#pragma unroll
+    for (int u = 0; u < CB; ++u) {
+      const int q = max(kt - u, 0);
+      d[u] = sd[q * 64];
+      xv[u] = KX ? sx[q * 64] : v.x[u];
+    }
+#pragma unroll
+    for (int u = 0; u < CB; ++u) {
+      const int q = kt - u;
+      if (q < nl - 1) d[u] = d[u] - v.cp[u] * dnext;
+      if (q >= 0) xo[(int64_t)q * plane + t] = xv[u] + omega * d[u];
+      dnext = d[u];
+    }
+  };
+  Back ba, bb;
+  bload(ba, nl - 1);
+  bload(bb, nl - 1 - CB);
+  int kt = nl - 1;
+  for (; kt >= CB; kt -= 2 * CB) {
+    bchunk(ba, kt);
+    bload(ba, kt - 2 * CB);
+    __builtin_amdgcn_sched_barrier(0);
+    bchunk(bb, kt - CB);
+    bload(bb, kt - 3 * CB);
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  if (kt >= 0) bchunk(ba, kt);
+}
+
 int lg2(int v) {
   int l = 0;
   while ((1 << l) < v) ++l;
@@ -574,9 +698,19 @@ void launch_smooth(hipStream_t s, lfr_mg* mg, lfr_mg_level& L, T* xo, const T* x
                          lg2(mg->nrhs), (T)L.sigma, (T)mg->omega, nbp);
     return;
   }
-  hipLaunchKernelGGL(k_mg_smooth<T>, dim3((unsigned)((n + bs - 1) / bs)), dim3(bs), 0, s, xo, xi, (const T*)L.b_d,
-                     (const T*)L.a_d, (const T*)L.d_d, (const T*)L.u_d, (const T*)L.cp_d, (const T*)L.iv_d,
-                     L.cell_next_d, L.ncell, mg->nl, lg2(mg->nrhs), (T)L.sigma, (T)mg->omega);
+  // x beside d' in LDS while that still leaves 8 waves a CU (µs a V-cycle with
+  // and without: C48L33 FP32 175 / 178, C12L10 FP64 87 / 90; at 30 KB C96L60
+  // FP32 1151 / 1115)
+  const size_t lds = (size_t)mg->nl * 64 * sizeof(T);
+  const unsigned nbp = ((unsigned)((n + 63) / 64) + 7u) & ~7u;
+  if (2 * lds <= 20 * 1024)
+    hipLaunchKernelGGL((k_mg_smooth_rt<T, true>), dim3(nbp), dim3(64), 2 * lds, s, xo, xi, (const T*)L.b_d,
+                       (const Band4<T>*)L.adui_d, (const T*)L.cp_d, L.cell_next_d, L.ncell, mg->nl, lg2(mg->nrhs),
+                       (T)L.sigma, (T)mg->omega, nbp);
+  else
+    hipLaunchKernelGGL((k_mg_smooth_rt<T, false>), dim3(nbp), dim3(64), lds, s, xo, xi, (const T*)L.b_d,
+                       (const Band4<T>*)L.adui_d, (const T*)L.cp_d, L.cell_next_d, L.ncell, mg->nl, lg2(mg->nrhs),
+                       (T)L.sigma, (T)mg->omega, nbp);
 }
 
 // two sweeps: x -> t -> x
@@ -659,7 +793,7 @@ int autotune(lfr_mg* mg) {
       return hipGetLastError() == hipSuccess ? LFR_OK : LFR_ERR_HIP;
     };
     L.block_smooth = cand[lfr_tune_pick(ctx, key, 3, 2, run)];
-    L.block_other = 256;
+    L.block_other = 256;   // (other layer counts smooth with one wave a workgroup)
   }
   return LFR_OK;
 }
@@ -817,18 +951,17 @@ int lfr_mg_solve(lfr_mg* mg, void* x_d, const void* b_d, int ncycles, double* re
   hipStream_t s = ctx->stream;
   const bool f32 = mg->prec == 4;
   const int R = mg->nrhs, lgR = lg2(R);
-  const size_t es = f32 ? 4 : 8;
-  int TC = (int)(32768 / ((size_t)mg->nl * R * es));
-  if (TC > 16) TC = 16;
-  if (TC < 1) TC = 1;
-  const size_t smem = (size_t)TC * mg->nl * R * es;
-  const unsigned gt = (unsigned)((F.ncell + TC - 1) / TC);
+  const int np = f32 ? kCvPairs<float> : kCvPairs<double>;
+  const unsigned gt = (unsigned)(((int64_t)F.ncell * R + np - 1) / np);
+  const size_t lcv = f32 ? convert_lds<float>(mg->nl, R) : convert_lds<double>(mg->nl, R);
+#define LFR_CV(T, TO, dst, src) \
+  hipLaunchKernelGGL((k_mg_convert<T, TO>), dim3(gt), dim3(256), lcv, s, (T*)(dst), (const T*)(src), F.ncell, mg->nl, lgR)
   if (f32) {
-    hipLaunchKernelGGL(k_to_mg<float>, dim3(gt), dim3(256), smem, s, (float*)F.b_d, (const float*)b_d, F.ncell, mg->nl, R, TC);
-    hipLaunchKernelGGL(k_to_mg<float>, dim3(gt), dim3(256), smem, s, (float*)F.x_d, (const float*)x_d, F.ncell, mg->nl, R, TC);
+    LFR_CV(float, true, F.b_d, b_d);
+    LFR_CV(float, true, F.x_d, x_d);
   } else {
-    hipLaunchKernelGGL(k_to_mg<double>, dim3(gt), dim3(256), smem, s, (double*)F.b_d, (const double*)b_d, F.ncell, mg->nl, R, TC);
-    hipLaunchKernelGGL(k_to_mg<double>, dim3(gt), dim3(256), smem, s, (double*)F.x_d, (const double*)x_d, F.ncell, mg->nl, R, TC);
+    LFR_CV(double, true, F.b_d, b_d);
+    LFR_CV(double, true, F.x_d, x_d);
   }
   LFR_CHECK_LAUNCH(ctx);
   if (!mg->graph) {
@@ -882,10 +1015,9 @@ int lfr_mg_solve(lfr_mg* mg, void* x_d, const void* b_d, int ncycles, double* re
       if (rc) return rc;
     }
   }
-  if (f32)
-    hipLaunchKernelGGL(k_from_mg<float>, dim3(gt), dim3(256), smem, s, (float*)x_d, (const float*)F.x_d, F.ncell, mg->nl, R, TC);
-  else
-    hipLaunchKernelGGL(k_from_mg<double>, dim3(gt), dim3(256), smem, s, (double*)x_d, (const double*)F.x_d, F.ncell, mg->nl, R, TC);
+  if (f32) LFR_CV(float, false, x_d, F.x_d);
+  else LFR_CV(double, false, x_d, F.x_d);
+#undef LFR_CV
   LFR_CHECK_LAUNCH(ctx);
   return LFR_OK;
 }

@@ -57,6 +57,20 @@ def test_vcycle_70_layers_bit_exact(ctx, prec, nrhs):
     np.testing.assert_allclose(res, reso, rtol=1e-12 if prec == 8 else 1e-5)
 
 
+@pytest.mark.parametrize("prec", [8, 4])
+@pytest.mark.parametrize("nrhs", [1, 8, 32])
+@pytest.mark.parametrize("nl", [2, 3, 4, 7, 8, 9, 16, 17, 33, 128])
+def test_vcycle_any_layer_count_bit_exact(ctx, prec, nl, nrhs):
+    """Layer counts around the smoother's chunks of 4 and 8 layers (one chunk,
+    whole ones, every remainder form, the tallest), x kept in LDS and read
+    again; 54 and 216 cells leave partial waves and partial conversion tiles."""
+    H = build_hierarchy((6, 3), nlayers=nl)
+    print(f"mg any nl={nl} prec={prec} nrhs={nrhs}", flush=True)
+    x, res, xo, reso = _run(ctx, H, prec, nrhs=nrhs, ncycles=1)
+    np.testing.assert_array_equal(x, xo)
+    np.testing.assert_allclose(res, reso, rtol=1e-12 if prec == 8 else 1e-5)
+
+
 def test_vcycle_options_and_repeat(ctx):
     """Other smoothing counts; a second solve replays the captured cycle."""
     H = build_hierarchy((8, 4, 2), nlayers=10)
