@@ -52,8 +52,9 @@ class Context:
 
     def sync_stream(self) -> None:
         """Queue subsequent library work on PyTorch's current stream."""
-        s = torch.cuda.current_stream(self.device).cuda_stream
-        check(lib().lfr_set_stream(self.h, _P(s)), self.h)
+        # the raw handle: a torch.cuda.Stream object a call costs more than the call
+        s = torch._C._cuda_getCurrentRawStream(self.device.index)
+        check(lib().lfr_set_stream(self.h, s), self.h)
 
     def synchronize(self) -> None:
         check(lib().lfr_synchronize(self.h), self.h)
@@ -110,15 +111,9 @@ class Space:
         check(lib().lfr_space_create(ctx.h, dm.ctypes.data_as(_P), fs.ndf, fs.ncells,
                                      fs.nlayers, fs.undf, C.byref(h)), ctx.h)
         self.h = h
+        self.undf: int = fs.undf
+        self.ndf: int = fs.ndf
         self._plans = {}
-
-    @property
-    def undf(self) -> int:
-        return self.fs.undf
-
-    @property
-    def ndf(self) -> int:
-        return self.fs.ndf
 
     def set_boundary(self, boundary=None) -> None:
         """Attach boundary_value(ndf, 2) (default: function_space.boundary_dofs)."""
@@ -186,13 +181,16 @@ class LMAOperator:
     _cache: dict = field(default_factory=dict)
 
     def __post_init__(self):
-        nt, nf = self.to_space.ndf, self.from_space.ndf
-        n3 = self.to_space.fs.ncell_3d
-        if tuple(self.matrix.shape) != (nf, nt, n3):
-            raise LfrError(1, f"operator matrix shape {tuple(self.matrix.shape)} != {(nf, nt, n3)}")
-        if not self.matrix.is_contiguous():
+        self.check_matrix(self.matrix)
+
+    def check_matrix(self, matrix: torch.Tensor) -> None:
+        """Raise unless ``matrix`` can stand in this operator's place."""
+        want = (self.from_space.ndf, self.to_space.ndf, self.to_space.fs.ncell_3d)
+        if tuple(matrix.shape) != want:
+            raise LfrError(1, f"operator matrix shape {tuple(matrix.shape)} != {want}")
+        if not matrix.is_contiguous():
             raise LfrError(1, "operator matrix must be contiguous")
-        if self.matrix.device != self.to_space.ctx.device:
+        if matrix.device != self.to_space.ctx.device:
             raise LfrError(1, "operator matrix on the wrong device")
 
     @property
