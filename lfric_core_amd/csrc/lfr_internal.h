@@ -70,14 +70,16 @@ struct lfr_space {
 // boundary values set).
 int lfr_enforce_bc_queue(lfr_ctx* ctx, int prec, void* field, const lfr_space* sp);
 
-// One class of output-dof columns with identical structure: every column has
-// `height` dofs and its contributions come from `ngroup` cells, each
-// contributing `gsize` local dofs (entries), listed in summation order.
+// One class of output-dof columns with the same structure: every column has
+// `height` dofs and its contributions come from (up to) `ngroup` cells, each
+// contributing (up to) `gsize` local dofs (entries), listed in summation order;
+// absent entries have code -1 and a valid cell.
 struct lfr_plan_class {
   int height = 0;
   int ngroup = 0;
   int gsize = 0;
   int ncol = 0;
+  bool absent = false;              // some entries are absent (code -1)
   int32_t* col_start_d = nullptr;   // (ncol) first dof of the column, 0-based
   int32_t* ent_d = nullptr;         // (ncol, ngroup*gsize, 2): cell (0-based), (i << 1) | shift
   // bundles of bsize columns (1 or 4) with the same cells and shifts, for

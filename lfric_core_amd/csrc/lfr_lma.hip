@@ -209,7 +209,7 @@ int run_bundles(lfr_ctx* ctx, const lfr_plan* plan, int kind, const T* M, const 
     b.nbund = c.nbund;
     b.H = c.height;
     b.ngroup = c.ngroup;
-    b.gs = c.gsize == 1 && c.height == nl ? 0 : c.gsize;
+    b.gs = c.gsize == 1 && c.height == nl && !c.absent ? 0 : c.gsize;
     b.nblocks = lfr_blocks((int64_t)c.nbund * c.height * (nf / (c.bsize == 4 ? F4 : F1)), kThreads);
     if (c.bsize == 4) {
       if (cl.n == lfr::kBunMaxClass) flush();
@@ -587,6 +587,26 @@ extern "C" int lfr_plan_create(lfr_ctx* ctx, const lfr_space* sp, const int32_t*
     by_sig[Sig(cols[ci].height, ngroup, gmax)].push_back((int)ci);
   }
 
+  // A class of few columns (the 8 cube corners of a vertex space, a limited
+  // area's boundary faces) joins the class of the same height and entries a
+  // cell whose columns have more cells, its missing cells as absent entries,
+  // which add nothing: a launch for it alone costs 6.6 µs (W0 C47L53), the
+  // entries it reads for nothing under a sixteenth of the larger class.
+  for (auto a = by_sig.begin(); a != by_sig.end();) {
+    auto into = by_sig.end();
+    for (auto b = by_sig.begin(); b != by_sig.end(); ++b)
+      if (std::get<0>(b->first) == std::get<0>(a->first) && std::get<2>(b->first) == std::get<2>(a->first) &&
+          std::get<1>(b->first) > std::get<1>(a->first) && a->second.size() * 16 <= b->second.size())
+        into = b;
+    if (into == by_sig.end()) {
+      ++a;
+      continue;
+    }
+    into->second.insert(into->second.end(), a->second.begin(), a->second.end());
+    std::sort(into->second.begin(), into->second.end());   // memory order
+    a = by_sig.erase(a);
+  }
+
   lfr_plan* plan = new lfr_plan();
   plan->uid = lfr_next_uid();
   plan->ctx = ctx;
@@ -615,11 +635,15 @@ extern "C" int lfr_plan_create(lfr_ctx* ctx, const lfr_space* sp, const int32_t*
         d[1] = (e.df << 1) | e.shift;
         ++slot;
       }
-      // padded slots keep the group's cell id and a negative code
+      // absent slots keep the group's cell id (an absent group the last one's)
+      // and a negative code
       for (int gg = 0; gg < pc.ngroup; ++gg)
         for (int s = 0; s < pc.gsize; ++s) {
           int32_t* d = &ent[(size_t)q * per + (size_t)(gg * pc.gsize + s) * 2];
-          if (d[1] < 0) d[0] = ent[(size_t)q * per + (size_t)(gg * pc.gsize) * 2];
+          if (d[1] < 0) {
+            d[0] = ent[(size_t)q * per + (size_t)(std::min(gg, g) * pc.gsize) * 2];
+            pc.absent = true;
+          }
         }
     }
     pc.starts_h = starts;

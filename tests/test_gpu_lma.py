@@ -189,3 +189,45 @@ def test_w2_mass_c96l70_fp32_bitexact(ctx):
     api.matrix_vector(y, _t(x, ctx), op, overwrite=True)
     torch.cuda.synchronize()
     np.testing.assert_array_equal(y.cpu().numpy(), ref)
+
+
+def _limited_area(n):
+    """n x n cells without neighbours past the edge."""
+    from lfric_core_amd.mesh import Mesh2D
+    c = np.arange(n * n).reshape(n, n)                       # rows from the north
+    nxt = np.zeros((n, n, 4), dtype=np.int32)                # W, S, E, N
+    nxt[:, 1:, 0] = c[:, :-1] + 1
+    nxt[:-1, :, 1] = c[1:] + 1
+    nxt[:, :-1, 2] = c[:, 1:] + 1
+    nxt[1:, :, 3] = c[:-1] + 1
+    v = np.arange((n + 1) * (n + 1)).reshape(n + 1, n + 1) + 1
+    vert = np.stack([v[1:, :-1], v[1:, 1:], v[:-1, 1:], v[:-1, :-1]], axis=-1)   # SW, SE, NE, NW
+    return Mesh2D("limited area", n * n, nxt.reshape(-1, 4), vert.reshape(-1, 4).astype(np.int32))
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("space,k,nl", [("W2", 0, 4), ("W2", 0, 5), ("W0", 0, 3), ("W0", 1, 2), ("W2", 1, 2)])
+def test_few_columns_join_a_larger_class(ctx, dtype, space, k, nl):
+    """A 72 x 72 limited area: the edge's columns, which fewer cells touch, are
+    a small part of all and take the larger class's kernel with absent
+    entries; matrix_vector and its transpose, packed and not, increment and
+    overwrite, bit for bit against the oracle."""
+    from lfric_core_amd import api
+    print(f"case absent entries {space} k={k} nl={nl} {dtype.__name__}", flush=True)
+    m = _limited_area(72)
+    fs, col = build_dofmap(m, space, nl, k), colour_cells(m)
+    sp = api.Space(ctx, fs)
+    st = Stream(91)
+    M = normal_lma(st, m.ncells * nl, fs.ndf, fs.ndf).astype(dtype)
+    x, y0 = st.uniform(fs.undf).astype(dtype), st.uniform(fs.undf).astype(dtype)
+    dev = lambda a: torch.from_numpy(a.copy()).to(ctx.device)
+    op = api.LMAOperator(dev(M), sp, sp, col)
+    for kind, call in ((0, api.matrix_vector), (1, api.transpose_matrix_vector)):
+        for over in (False, True):
+            start = np.zeros_like(y0) if over else y0.copy()
+            ref = oracle.invoke_coloured(kind, col, nl, start, x, M, fs.dofmap, fs.dofmap)
+            y = call(dev(y0), dev(x), op, overwrite=over)
+            np.testing.assert_array_equal(y.cpu().numpy(), ref)
+            if k == 0:
+                y = api.PackedOperator(op, kind).apply(dev(y0), dev(x), overwrite=over)
+                np.testing.assert_array_equal(y.cpu().numpy(), ref)
