@@ -7,9 +7,9 @@
 //
 //   apply    z = A p            gather pass, fused partial sums of <p, z>
 //   alpha    alpha = rz / <p,z> one block, fixed-order combine of partials
-//   update   x += alpha p, r -= alpha z (, z = r / diag), partials of <r,r>, <r,z>
-//   beta     ||r||, convergence test, beta = rz_new / rz
-//   direction p = z + beta p
+//   update   r -= alpha z (, z = r / diag), partials of <r,r>, <r,z>
+//   direction ||r||, convergence test, beta = rz_new / rz,
+//            x += alpha p, p = z + beta p
 //
 // The scalars never leave the device.  The convergence predicate is
 // evaluated on the device; once it holds every later kernel returns at
@@ -34,8 +34,11 @@ namespace {
 
 using lfr::kThreads;
 
-enum Slot { S_STOP = 0, S_RZ, S_ALPHA, S_BETA, S_RNRM0, S_RNRM, S_ITER, S_NAN, S_RR, S_NSLOT = 16 };
+enum Slot { S_STOP = 0, S_RZ, S_ALPHA, S_BETA, S_RNRM0, S_RNRM, S_ITER, S_NAN, S_RR, S_HALT, S_NSLOT = 16 };
 // S_STOP: 0 running, 1 converged, 2 max_iter reached, 3 NaN
+// S_HALT: S_STOP as the last k_cg_alpha saw it.  k_cg_beta_direction sets
+// S_STOP while others of its workgroups have yet to start, and those still
+// have their part of x to update, so that kernel looks at S_HALT.
 
 constexpr double kEps = 2.220446049250313e-16;  // epsilon(1.0_r_def), constants_mod.F90:167
 
@@ -52,9 +55,13 @@ constexpr int kAlphaThreads = 1024;
 __global__ void __launch_bounds__(kAlphaThreads)
 k_cg_alpha(const double* __restrict__ part, int np, const double* __restrict__ part_rz, int nrz,
            double* __restrict__ S, int max_iter) {
-  if (S[S_STOP] != 0.0) return;
-  if (S[S_ITER] >= (double)max_iter) {
-    if (threadIdx.x == 0) S[S_STOP] = 2.0;
+  const double halt = S[S_STOP] != 0.0 ? S[S_STOP] : (S[S_ITER] >= (double)max_iter ? 2.0 : 0.0);
+  if (halt != 0.0) {
+    __syncthreads();   // every thread has read S_STOP
+    if (threadIdx.x == 0) {
+      S[S_STOP] = halt;
+      S[S_HALT] = halt;
+    }
     return;
   }
   __shared__ double lds[kAlphaThreads / 64];
@@ -73,29 +80,45 @@ k_cg_alpha(const double* __restrict__ part, int np, const double* __restrict__ p
   }
 }
 
+// Strides of the grid a trip of the two CG vector passes takes: the loads of
+// all of them are issued before the first is used (at clamped addresses, so
+// that none sits behind a branch), the order of every sum is unchanged.
+constexpr int kCgUnroll = 4;
+
+// r = r - alpha A p (z holds A p) with the partials of <r, r>; with a
+// diagonal, z = r / diag with those of <r, z>.
 template <typename T, bool DIAG>
 __global__ void __launch_bounds__(kThreads)
-k_cg_update(T* __restrict__ x, T* __restrict__ r, const T* __restrict__ p, T* __restrict__ z,
-            const T* __restrict__ diag, int64_t n, const double* __restrict__ S,
-            double* __restrict__ part_rr, double* __restrict__ part_rz) {
+k_cg_update(T* __restrict__ r, T* __restrict__ z, const T* __restrict__ diag, int64_t n,
+            const double* __restrict__ S, double* __restrict__ part_rr, double* __restrict__ part_rz) {
   if (S[S_STOP] != 0.0) return;
   __shared__ double lds[kThreads / 64];
-  const double alpha = S[S_ALPHA];
-  const T a = (T)alpha, ma = (T)(-alpha);
+  const T ma = (T)(-S[S_ALPHA]);
   double rr = 0.0, rz = 0.0;
-  for (int64_t i = (int64_t)blockIdx.x * kThreads + threadIdx.x; i < n;
-       i += (int64_t)gridDim.x * kThreads) {
-    const T xp = a * p[i];
-    x[i] = x[i] + xp;
-    const T rq = ma * z[i];
-    const T ri = r[i] + rq;
-    r[i] = ri;
-    const double rd = (double)ri;
-    rr = rr + rd * rd;
-    if (DIAG) {
-      const T zi = ri / diag[i];
-      z[i] = zi;
-      rz = rz + rd * (double)zi;
+  const int64_t st = (int64_t)gridDim.x * kThreads;
+  for (int64_t i = (int64_t)blockIdx.x * kThreads + threadIdx.x; i < n; i += kCgUnroll * st) {
+    T rv[kCgUnroll], zv[kCgUnroll], dv[kCgUnroll];
+#pragma unroll
+    for (int q = 0; q < kCgUnroll; ++q) {
+      const int64_t j = i + q * st < n ? i + q * st : i;
+      rv[q] = r[j];
+      zv[q] = z[j];
+      dv[q] = DIAG ? diag[j] : T(1);
+    }
+#pragma unroll
+    for (int q = 0; q < kCgUnroll; ++q) {
+      const int64_t j = i + q * st;
+      if (j >= n) break;
+      const T rq = ma * zv[q];
+      const T ri = rv[q] + rq;
+      r[j] = ri;
+      const double rd = (double)ri;
+      rr = rr + rd * rd;
+      if (DIAG) {
+        const T zi = ri / dv[q];
+        z[j] = zi;
+        rz = rz + rd * (double)zi;
+      }
     }
   }
   rr = lfr::block_sum(rr, lds);
@@ -106,17 +129,26 @@ k_cg_update(T* __restrict__ x, T* __restrict__ r, const T* __restrict__ p, T* __
   }
 }
 
-// beta and the convergence test, then p = beta * p + z.  Every workgroup
-// sums the update's partials in the same order (identical bits); workgroup 0
-// records the results; S_RZ (read here) is only written by k_cg_alpha.
+// x = x + alpha p, beta and the convergence test, then p = beta * p + z
+// unless the test stops the solve.  x takes its step here, where p is read
+// anyway, and not with r: an iteration is then 8 vector passes, not 9.  x is
+// not wanted again for a whole iteration, so it streams past the caches
+// (non-temporal) and leaves them to p and r, which the apply and the next
+// update read.  C96L70 solves: FP64 to 1e-10 16.35 -> 15.51 ms (15.89 without
+// the non-temporal x, 15.8 with one stride a trip), refined 9.68 -> 9.63 ms
+// (9.76; 10.4).
+// Every workgroup sums the update's partials in the same order (identical
+// bits); workgroup 0 records the results; S_RZ (read here) is only written
+// by k_cg_alpha.
 template <typename T>
 __global__ void __launch_bounds__(kThreads)
-k_cg_beta_direction(T* __restrict__ p, const T* __restrict__ z, int64_t n, const double* __restrict__ part_rr,
-                    const double* __restrict__ part_rz, int np, double* __restrict__ S, int monitor, double r_tol,
-                    double a_tol, int diag) {
-  if (S[S_STOP] != 0.0) return;
+k_cg_beta_direction(T* __restrict__ x, T* __restrict__ p, const T* __restrict__ z, int64_t n,
+                    const double* __restrict__ part_rr, const double* __restrict__ part_rz, int np,
+                    double* __restrict__ S, int monitor, double r_tol, double a_tol, int diag) {
+  if (S[S_HALT] != 0.0) return;
   __shared__ double lds[kThreads / 64];
   __shared__ double bc[2];
+  const T a = (T)S[S_ALPHA];
   const double srr = lfr::strided_sum(part_rr, np);
   const double srz = diag ? lfr::strided_sum(part_rz, np) : 0.0;
   const double rr = lfr::block_sum(srr, lds);
@@ -139,12 +171,27 @@ k_cg_beta_direction(T* __restrict__ p, const T* __restrict__ z, int64_t n, const
     bc[1] = beta;
   }
   __syncthreads();
-  if (bc[0] != 0.0) return;
+  const bool go = bc[0] == 0.0;
   const T b = (T)bc[1];
-  for (int64_t i = (int64_t)blockIdx.x * kThreads + threadIdx.x; i < n;
-       i += (int64_t)gridDim.x * kThreads) {
-    const T bp = b * p[i];
-    p[i] = bp + z[i];
+  const int64_t st = (int64_t)gridDim.x * kThreads;
+  for (int64_t i = (int64_t)blockIdx.x * kThreads + threadIdx.x; i < n; i += kCgUnroll * st) {
+    T xv[kCgUnroll], pv[kCgUnroll], zv[kCgUnroll];
+#pragma unroll
+    for (int q = 0; q < kCgUnroll; ++q) {
+      const int64_t j = i + q * st < n ? i + q * st : i;
+      xv[q] = __builtin_nontemporal_load(x + j);
+      pv[q] = p[j];
+      zv[q] = z[j];
+    }
+#pragma unroll
+    for (int q = 0; q < kCgUnroll; ++q) {
+      const int64_t j = i + q * st;
+      if (j >= n) break;
+      const T xp = a * pv[q];
+      __builtin_nontemporal_store(xv[q] + xp, x + j);
+      const T bp = b * pv[q];
+      if (go) p[j] = bp + zv[q];
+    }
   }
 }
 
@@ -664,12 +711,12 @@ int cg_iterations(lfr_ctx* ctx, const lfr_lma_op* A, const lfr_solver_params* P,
     hipLaunchKernelGGL(k_cg_alpha, dim3(1), dim3(kAlphaThreads), 0, ctx->stream, w.part_apply,
                        np_apply, diag ? w.part_rz : w.part_rr, G, w.S, P->max_iter);
     if (diag)
-      hipLaunchKernelGGL((k_cg_update<T, true>), dim3(G), dim3(kThreads), 0, ctx->stream, x, r, p,
-                         z, dg, n, w.S, w.part_rr, w.part_rz);
+      hipLaunchKernelGGL((k_cg_update<T, true>), dim3(G), dim3(kThreads), 0, ctx->stream, r, z, dg,
+                         n, w.S, w.part_rr, w.part_rz);
     else
-      hipLaunchKernelGGL((k_cg_update<T, false>), dim3(G), dim3(kThreads), 0, ctx->stream, x, r,
-                         p, z, dg, n, w.S, w.part_rr, w.part_rz);
-    hipLaunchKernelGGL(k_cg_beta_direction<T>, dim3(G), dim3(kThreads), 0, ctx->stream, p,
+      hipLaunchKernelGGL((k_cg_update<T, false>), dim3(G), dim3(kThreads), 0, ctx->stream, r, z, dg,
+                         n, w.S, w.part_rr, w.part_rz);
+    hipLaunchKernelGGL(k_cg_beta_direction<T>, dim3(G), dim3(kThreads), 0, ctx->stream, x, p,
                        diag ? (const T*)z : (const T*)r, n, w.part_rr, w.part_rz, G, w.S,
                        P->monitor_convergence, P->r_tol, P->a_tol, (int)diag);
     LFR_CHECK_LAUNCH(ctx);

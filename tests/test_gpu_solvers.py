@@ -216,3 +216,37 @@ def test_cg_repeated_solves_and_fixed_counts(ctx, prob):
     x = torch.zeros_like(b)
     ConjugateGradient(op, max_iter=res[0][0], monitor_convergence=False).apply(x, b, x_is_zero=True)
     np.testing.assert_array_equal(x.cpu().numpy(), res[0][1])
+
+
+@pytest.mark.parametrize("edge,nlayers", [(2, 3), (8, 10), (11, 7)])
+@pytest.mark.parametrize("diag", [False, True])
+def test_cg_x_has_every_step_up_to_the_stop(ctx, edge, nlayers, diag):
+    """x holds exactly the steps up to the stopping one, wherever in a queued
+    run of iterations the tolerance or max_iter stops it, on grids whose last
+    workgroup has fewer dofs than its strides (FP64; the oracle's dot products
+    sum in another order: 1e-11 relative)."""
+    from lfric_core_amd import api
+    from lfric_core_amd.solvers import ConjugateGradient, DiagonalPreconditioner
+    print(f"case cg stops C{edge}L{nlayers} diag={diag}", flush=True)
+    cfg = precision_config(edge, nlayers, with_div_grad=False)
+    w2 = api.Space(ctx, cfg.w2)
+    op = _op(ctx, cfg, w2, np.float64)
+    A = _oracle_apply(cfg, cfg.mass)
+    d = 6.0 + np.abs(cfg.b)
+    prec = (lambda v: v / d) if diag else None
+    pre = DiagonalPreconditioner(torch.from_numpy(d).to(ctx.device)) if diag else None
+    b = torch.from_numpy(cfg.b).to(ctx.device)
+    ratio = 1.0
+    for it in range(1, 7):
+        xo = np.zeros(cfg.w2.undf)
+        _, _, r0, rn = cg_solve(A, xo, cfg.b, prec=prec, max_iter=it, monitor=False)
+        if not rn / r0 < 0.9 * ratio:
+            continue
+        for by_tol in (False, True):
+            # a tolerance between this residual and the smallest so far, or max_iter
+            tol = dict(r_tol=0.5 * (rn / r0 + ratio), max_iter=50) if by_tol else dict(r_tol=1e-14, max_iter=it)
+            x = torch.zeros(cfg.w2.undf, dtype=torch.float64, device=ctx.device)
+            st = (ConjugateGradient(op, pre, **tol) if diag else ConjugateGradient(op, **tol)).apply(x, b)
+            assert st.iterations == it and bool(st.converged) == by_tol
+            assert np.linalg.norm(x.cpu().numpy() - xo) <= 1e-11 * np.linalg.norm(xo)
+        ratio = rn / r0
