@@ -479,15 +479,17 @@ k_gather_vec(const T* __restrict__ M, const T* __restrict__ x, T* __restrict__ y
 // One launch takes all classes of a plan with four rows a bundle: their
 // blocks are interleaved chunk by chunk so that the blocks in flight belong to
 // the same few cells and find their operand in L2 (a launch a class reads the
-// operand from HBM once per class: 3316 against 2520 µs below).  The fields of
+// operand from HBM once per class: 3316 against 2526 µs).  The fields of
 // a level are read in 16-byte pieces that lie side by side across its lanes.
 // Measured, W2 order 1 (36 x 36), a row a thread -> this form: 16 fields FP64
-// C32L70 6060 -> 2520 µs, FP32 C24L33 1155 -> 332 µs, one field FP64 C32L70
+// C32L70 6060 -> 2240-2300 µs, FP32 C24L33 1155 -> 317 µs, one field FP64 C32L70
 // 1290 -> 850-990 µs (4.7-5.5 TB/s), FP32 990 -> 520 µs.  What bounds the 16
-// fields now is L1 (two of three accesses are the operand and the rows'
-// matrix values) and the 8 wavefronts a CU that its registers leave; two
-// fields a thread (more wavefronts) took 2970 µs, streaming matrix loads
-// 2620, a whole dofmap vector per load 2650.
+// fields now is memory latency: 8 wavefronts a CU (their registers leave no
+// more) with two blocks of input dofs in flight; the caches move 14 GB a pass
+// at 6 TB/s, twice the least, as each bundle reads its cells' operand again.
+// Two fields a thread (more wavefronts) took 2970 µs, non-temporal matrix
+// loads 2550 (rows of levels straddle cache lines), bundles in tiles of cells
+// 2150-2200.
 // ---------------------------------------------------------------------------
 struct BunClass {
   const int32_t* bund;
@@ -644,33 +646,28 @@ __device__ __forceinline__ void gather_bun_body(const T* __restrict__ M, const T
 }
 
 // The same for four rows and ndata a multiple of 4: the four lanes of a quad
-// hold the fields of one level, so each loads the matrix values of one of the
-// four rows and the others take them by a quad broadcast.  One load
-// instruction then brings four rows' values and a lane keeps a quarter of
-// them, which leaves registers for a block of U input dofs in flight ahead of
-// the one being summed (across the cells of a column too).
-template <int I, typename T>
-__device__ __forceinline__ T quad_bcast(T v) {
-  constexpr int ctrl = I * 0x55;   // every lane of the quad reads lane I
-  if constexpr (sizeof(T) == 4) {
-    return __builtin_bit_cast(T, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), ctrl, 0xf, 0xf, true));
-  } else {
-    struct I2 {
-      int a, b;
-    };
-    I2 i = __builtin_bit_cast(I2, v);
-    i.a = __builtin_amdgcn_mov_dpp(i.a, ctrl, 0xf, 0xf, true);
-    i.b = __builtin_amdgcn_mov_dpp(i.b, ctrl, 0xf, 0xf, true);
-    return __builtin_bit_cast(T, i);
-  }
-}
-
+// hold the fields of one level, a wavefront the levels of 16 quads.  The
+// matrix values of a wavefront's 4 rows x 16 levels come by one load an input
+// dof, lane (row, quad) = (lane >> 4, lane & 15), so that neighbouring lanes
+// read neighbouring levels (one cache access where each of the quad's lanes
+// reading a row of its own made four), and go to the quads through LDS; the
+// dof numbers of a block of input dofs come by one load and a shuffle.  16
+// fields FP64 C32L70: 2526 µs with a row a lane and a quad broadcast -> 2389
+// with this split -> 2300 with the matrix values two blocks ahead and the dof
+// numbers ahead of the operand, so that no step waits for its own loads
+// (2240-2300 from run to run with the last blocks peeled).
+// A lane keeps a quarter of the matrix values, which leaves registers for a
+// block of U input dofs in flight ahead of the one being summed (across the
+// cells of a column too).
 template <typename T, int F, int GS, int KIND, bool MASK>
 __device__ __forceinline__ void gather_quad_body(const T* __restrict__ M, const T* __restrict__ x, T* __restrict__ y,
                                                  const int32_t* __restrict__ map_in, const BunClass& bc, unsigned blk,
-                                                 int nl, int64_t n3, int ndf_out, int ndf_in, int nf, int overwrite) {
+                                                 int nl, int64_t n3, int ndf_out, int ndf_in, int nf, int overwrite,
+                                                 T* __restrict__ lm) {
   constexpr int R = 4;
-  constexpr int U = GS == 2 ? 2 : 4;
+  // input dofs a block: fewer where the sums of two entries, or of an entry
+  // and its cell (kind 1), leave no registers for more
+  constexpr int U = KIND == 1 && F >= 3 ? (GS == 2 ? 1 : 2) : (GS == 2 ? 2 : 4);
   constexpr int PF = F * (int)sizeof(T) <= 16 ? F : (F % 2 == 0 ? 2 : 1);   // fields side by side in a lane
   constexpr int P = F / PF;
   const int ng = nf / F, ngroup = bc.ngroup, H = bc.H;
@@ -711,57 +708,108 @@ __device__ __forceinline__ void gather_quad_body(const T* __restrict__ M, const 
   };
   if (KIND == 1) zero_dot();
   const int64_t js = KIND == 0 ? n3 * ndf_out : n3;   // one input dof further
-  // the load cursor: input dofs jl.. of group gl
-  int gl = 0, jl = 0;
-  const int32_t* mi;
-  const T *pm[GS], *px[GS];
-  const auto enter = [&] {
-    const int32_t* e = rec + R + gl * (1 + GS * R);
-    const int cc = e[0];
-    mi = map_in + (int64_t)cc * ndf_in;
+  // what this lane loads for the wavefront: row lrow of quad lquad's level
+  // (of the first level where that quad is past the end, as above)
+  const int lane = threadIdx.x & 63, quad = lane >> 2, lquad = lane & 15, lrow = lane >> 4;
+  const int64_t tq = t - lane + 4 * lquad;
+  const int64_t slotq = tq < (int64_t)bc.nbund * H * ng ? tq / ng : 0;
+  const int bq = (int)(slotq / H);
+  const int Lq = (int)(slotq - (int64_t)bq * H);
+  const int32_t* recq = bc.bund + (int64_t)bq * (R + ngroup * (1 + GS * R));
+  // the dof cursor, a block ahead of the operand's: lane (u, quad) loads the
+  // dof number jd + u of the quad's cell in group gd
+  int gd = 0, jd = 0;
+  const int32_t* mi = map_in + (int64_t)recq[R] * ndf_in;
+  const auto dofs = [&]() -> int {
+    const int d = mi[min(jd + min(lrow, U - 1), ndf_in - 1)];
+    jd += U;
+    if (jd >= ndf_in && gd + 1 < ngroup) {
+      ++gd;
+      jd = 0;
+      mi = map_in + (int64_t)recq[R + gd * (1 + GS * R)] * ndf_in;
+    }
+    return d;
+  };
+  // the operand's cursor: input dofs jx.. of group gx
+  int gx = 0, jx = 0;
+  const T* px[GS];
+  const auto enter_x = [&] {
 #pragma unroll
     for (int q = 0; q < GS; ++q) {
-      const int code = e[1 + q * R + (threadIdx.x & 3)];
-      const int k = L - (code & 1);
-      const int kk = k < 0 ? 0 : (k >= nl ? nl - 1 : k);   // clamped: always in bounds
-      const int64_t i = code >= 0 ? (code >> 1) : 0;
+      const int k = L - (rec[R + gx * (1 + GS * R) + 1 + q * R] & 1);   // a bundle's rows have one shift
+      const int kk = k < 0 ? 0 : (k >= nl ? nl - 1 : k);                // clamped: always in bounds
       px[q] = x + (int64_t)kk * nf + r0;
-      pm[q] = M + (int64_t)cc * nl + kk + n3 * (KIND == 0 ? i : i * ndf_in);
     }
   };
-  struct Block {
-    T m[GS][U], xv[GS][U][F];
+  struct Operand {
+    T v[GS][U][F];
   };
-  const auto load = [&](Block& v) {
+  // past the last group a cursor stays on its last block (in bounds, unused)
+  const auto load_x = [&](Operand& o, int d) {
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      const int j = min(jl + u, ndf_in - 1);
-      const int64_t xb = (int64_t)mi[j] * nf;
+      const int64_t xb = (int64_t)__shfl(d, 16 * u + quad) * nf;
 #pragma unroll
       for (int q = 0; q < GS; ++q) {
-        v.m[q][u] = pm[q][js * j];
 #pragma unroll
         for (int p = 0; p < P; ++p) {
           const LVec<T, PF> w = ldvec<T, PF, false>(px[q] + xb + p * ps);
 #pragma unroll
-          for (int f = 0; f < PF; ++f) v.xv[q][u][p * PF + f] = w.v[f];
+          for (int f = 0; f < PF; ++f) o.v[q][u][p * PF + f] = w.v[f];
         }
       }
     }
-    // past the last group the cursor stays on its last block (in bounds, unused)
-    jl += U;
-    if (jl >= ndf_in && gl + 1 < ngroup) {
-      ++gl;
-      jl = 0;
-      enter();
+    jx += U;
+    if (jx >= ndf_in && gx + 1 < ngroup) {
+      ++gx;
+      jx = 0;
+      enter_x();
     }
   };
-  bool ok[GS];
-  const auto one = [&](const Block& v, int u) {
+  // the matrix's cursor: input dofs jm.. of group gm
+  int gm = 0, jm = 0;
+  const T* pm[GS];
+  const auto enter_m = [&] {
+    const int32_t* e = recq + R + gm * (1 + GS * R);
 #pragma unroll
     for (int q = 0; q < GS; ++q) {
-      const T m[R] = {quad_bcast<0>(v.m[q][u]), quad_bcast<1>(v.m[q][u]), quad_bcast<2>(v.m[q][u]),
-                      quad_bcast<3>(v.m[q][u])};
+      const int code = e[1 + q * R + lrow];
+      const int k = Lq - (code & 1);
+      const int kk = k < 0 ? 0 : (k >= nl ? nl - 1 : k);
+      const int64_t i = code >= 0 ? (code >> 1) : 0;
+      pm[q] = M + (int64_t)e[0] * nl + kk + n3 * (KIND == 0 ? i : i * ndf_in);
+    }
+  };
+  struct Rows {
+    T v[GS][U];
+  };
+  const auto load_m = [&](Rows& m) {
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+#pragma unroll
+      for (int q = 0; q < GS; ++q) m.v[q][u] = pm[q][js * min(jm + u, ndf_in - 1)];
+    jm += U;
+    if (jm >= ndf_in && gm + 1 < ngroup) {
+      ++gm;
+      jm = 0;
+      enter_m();
+    }
+  };
+  // (a wavefront's LDS accesses take effect in order, and lm is its own)
+  const auto share = [&](const Rows& m) {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+#pragma unroll
+    for (int q = 0; q < GS; ++q)
+#pragma unroll
+      for (int u = 0; u < U; ++u) lm[(q * U + u) * 64 + 4 * lquad + lrow] = m.v[q][u];
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  };
+  bool ok[GS];
+  const auto one = [&](const Operand& o, int u) {
+#pragma unroll
+    for (int q = 0; q < GS; ++q) {
+      const T* lr = lm + (q * U + u) * 64 + 4 * quad;
+      const T m[R] = {lr[0], lr[1], lr[2], lr[3]};
       if (KIND == 0) {
         // df2 outer, df inner; an entry without a layer here adds nothing
         if (ok[q]) {
@@ -769,7 +817,7 @@ __device__ __forceinline__ void gather_quad_body(const T* __restrict__ M, const 
           for (int r = 0; r < R; ++r)
 #pragma unroll
             for (int f = 0; f < F; ++f) {
-              const T p = m[r] * v.xv[q][u][f];
+              const T p = m[r] * o.v[q][u][f];
               acc[r][f] = acc[r][f] + p;
             }
         }
@@ -778,7 +826,7 @@ __device__ __forceinline__ void gather_quad_body(const T* __restrict__ M, const 
         for (int r = 0; r < R; ++r)
 #pragma unroll
           for (int f = 0; f < F; ++f) {
-            const T p = m[r] * v.xv[q][u][f];
+            const T p = m[r] * o.v[q][u][f];
             dot[q][r][f] = dot[q][r][f] + p;
           }
       }
@@ -794,14 +842,14 @@ __device__ __forceinline__ void gather_quad_body(const T* __restrict__ M, const 
       ok[q] = !MASK || (c0 >= 0 && k >= 0 && k < nl);
     }
   };
-  const auto sum = [&](const Block& v) {
+  const auto sum = [&](const Operand& o) {
     if (j + U <= ndf_in) {
 #pragma unroll
-      for (int u = 0; u < U; ++u) one(v, u);
+      for (int u = 0; u < U; ++u) one(o, u);
     } else {
 #pragma unroll
       for (int u = 0; u < U; ++u)
-        if (j + u < ndf_in) one(v, u);
+        if (j + u < ndf_in) one(o, u);
     }
     j += U;
     if (j >= ndf_in) {
@@ -821,21 +869,41 @@ __device__ __forceinline__ void gather_quad_body(const T* __restrict__ M, const 
       if (MASK && g < ngroup) mask();
     }
   };
-  enter();
+  // Block i is summed while the operand of block i + 1 and the matrix values
+  // of blocks i + 1 and i + 2 are in flight; loads complete in order, so each
+  // step issues first what the next one needs first.
+  enter_x();
+  enter_m();
   mask();
-  Block va, vb;
-  load(va);
+  Operand xa, xb;
+  Rows ma, mb;
+  int da = dofs(), db = dofs();
+  load_x(xa, da);
+  load_m(ma);
+  load_m(mb);
+  const auto step = [&](const Operand& now, Operand& next, Rows& m, int& d, int& dn) {
+    share(m);
+    d = dofs();
+    load_x(next, dn);
+    load_m(m);
+    __builtin_amdgcn_sched_barrier(0);
+    sum(now);
+  };
   const int nblk = ngroup * ((ndf_in + U - 1) / U);
   int i = 0;
-  for (; i + 1 < nblk; i += 2) {
-    load(vb);
-    __builtin_amdgcn_sched_barrier(0);
-    sum(va);
-    load(va);
-    __builtin_amdgcn_sched_barrier(0);
-    sum(vb);
+  for (; i + 2 < nblk; i += 2) {
+    step(xa, xb, ma, da, db);
+    step(xb, xa, mb, db, da);
   }
-  if (i < nblk) sum(va);
+  share(ma);
+  if (i + 1 < nblk) {
+    load_x(xb, db);
+    sum(xa);
+    share(mb);
+    sum(xb);
+  } else {
+    sum(xa);
+  }
   if (valid) {
 #pragma unroll
     for (int r = 0; r < R; ++r) {
@@ -875,6 +943,9 @@ k_gather_bun(const T* __restrict__ M, const T* __restrict__ x, T* __restrict__ y
   while (k > 0 && start(k) > lb) --k;
   while (k + 1 < cl.nchunk && start(k + 1) <= lb) ++k;
   unsigned rest = lb - start(k);
+  // a wavefront's matrix values of one block of input dofs (gather_quad_body)
+  __shared__ __attribute__((aligned(16))) T lds[QUAD ? kThreads / 64 * 256 : 1];
+  T* lm = lds + (QUAD ? (threadIdx.x >> 6) * 256 : 0);
   for (int c = 0; c < cl.n; ++c) {
     const unsigned f = bun_first(k, cl.c[c].nblocks, cl.nchunk);
     const unsigned m = bun_first(k + 1, cl.c[c].nblocks, cl.nchunk) - f;
@@ -882,18 +953,24 @@ k_gather_bun(const T* __restrict__ M, const T* __restrict__ x, T* __restrict__ y
       const BunClass& bc = cl.c[c];
       if constexpr (QUAD) {
         if (bc.gs == 0)
-          gather_quad_body<T, F, 1, KIND, false>(M, x, y, map_in, bc, f + rest, nl, n3, ndf_out, ndf_in, nf, overwrite);
+          gather_quad_body<T, F, 1, KIND, false>(M, x, y, map_in, bc, f + rest,
+              nl, n3, ndf_out, ndf_in, nf, overwrite, lm);
         else if (bc.gs == 1)
-          gather_quad_body<T, F, 1, KIND, true>(M, x, y, map_in, bc, f + rest, nl, n3, ndf_out, ndf_in, nf, overwrite);
+          gather_quad_body<T, F, 1, KIND, true>(M, x, y, map_in, bc, f + rest,
+              nl, n3, ndf_out, ndf_in, nf, overwrite, lm);
         else
-          gather_quad_body<T, F, 2, KIND, true>(M, x, y, map_in, bc, f + rest, nl, n3, ndf_out, ndf_in, nf, overwrite);
+          gather_quad_body<T, F, 2, KIND, true>(M, x, y, map_in, bc, f + rest,
+              nl, n3, ndf_out, ndf_in, nf, overwrite, lm);
       } else {
         if (bc.gs == 0)
-          gather_bun_body<T, 4, F, 1, KIND, false>(M, x, y, map_in, bc, f + rest, nl, n3, ndf_out, ndf_in, nf, overwrite);
+          gather_bun_body<T, 4, F, 1, KIND, false>(M, x, y, map_in, bc, f + rest,
+              nl, n3, ndf_out, ndf_in, nf, overwrite);
         else if (bc.gs == 1)
-          gather_bun_body<T, 4, F, 1, KIND, true>(M, x, y, map_in, bc, f + rest, nl, n3, ndf_out, ndf_in, nf, overwrite);
+          gather_bun_body<T, 4, F, 1, KIND, true>(M, x, y, map_in, bc, f + rest,
+              nl, n3, ndf_out, ndf_in, nf, overwrite);
         else
-          gather_bun_body<T, 4, F, 2, KIND, true>(M, x, y, map_in, bc, f + rest, nl, n3, ndf_out, ndf_in, nf, overwrite);
+          gather_bun_body<T, 4, F, 2, KIND, true>(M, x, y, map_in, bc, f + rest,
+              nl, n3, ndf_out, ndf_in, nf, overwrite);
       }
       return;
     }

@@ -127,3 +127,29 @@ def test_bundled_applies_bitexact(ctx, dtype, space, k, nl):
                     single(ys, _t(xr, ctx), op, overwrite=True)
                     torch.cuda.synchronize()
                     np.testing.assert_array_equal(ys.cpu().numpy(), ref)
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("nl", [15, 16, 17, 33])
+def test_quads_across_bundles_bitexact(ctx, dtype, nl):
+    """A wavefront of quads loads 16 levels' matrix values for all its lanes:
+    columns of just under, exactly and just over 16 levels (a wavefront then
+    holds levels of one bundle or of two, at any offset), both kinds, against
+    the oracle."""
+    from lfric_core_amd import api
+    m, col, fs, sp = _setup(ctx, 2, nl, 1, {"W2"})
+    fs, sp = fs["W2"], sp["W2"]
+    st = Stream(34)
+    M = normal_lma(st, m.ncells * nl, fs.ndf, fs.ndf).astype(dtype)
+    op = api.LMAOperator(_t(M, ctx), sp, sp, col)
+    for nd in (4, 16, 24):
+        print(f"case quads nl={nl} nd={nd} {dtype.__name__}", flush=True)
+        X = st.uniform(fs.undf * nd).reshape(fs.undf, nd).astype(dtype)
+        for kind in (0, 1):
+            y = torch.full((fs.undf, nd), float("nan"), dtype=op.matrix.dtype, device=ctx.device)
+            api.matrix_vector_ndata(y, _t(X, ctx), op, overwrite=True, transpose=kind == 1)
+            torch.cuda.synchronize()
+            for r in (0, nd - 1):
+                ref = oracle.invoke_coloured(kind, col, nl, np.zeros(fs.undf, dtype), np.ascontiguousarray(X[:, r]), M,
+                                             fs.dofmap, fs.dofmap)
+                np.testing.assert_array_equal(y[:, r].cpu().numpy(), ref)
