@@ -38,7 +38,11 @@ def _prec(t: torch.Tensor) -> int:
 
 
 class Context:
-    """A device context (lfr_init); work is queued on PyTorch's current stream."""
+    """A device context (lfr_init); work is queued on PyTorch's current stream.
+
+    A context serves one call at a time: threads that call concurrently have a
+    context each (the stream of a launch is set in a call of its own before it).
+    """
 
     def __init__(self, device: int = 0):
         if not torch.cuda.is_available():
@@ -214,18 +218,48 @@ def _field(t: torch.Tensor, space: Space, name: str, dtype=None) -> None:
         raise LfrError(1, f"{name} dtype {t.dtype} differs from the operator's {dtype}")
 
 
-def matrix_vector(lhs: torch.Tensor, x: torch.Tensor, op: LMAOperator, overwrite: bool = False):
-    """lhs += M x (GH_INC, colour order); overwrite=True gives lhs = M x."""
+# The applies with another matrix of the operator's shape in its place, on
+# checked outputs: api and autograd both queue through these, so that each
+# launch's stream is set right before it, whatever another thread has set on
+# the context since the launch before (building a plan or a buffer in between
+# lets other threads run).
+
+def _matrix_vector(lhs: torch.Tensor, x: torch.Tensor, matrix: torch.Tensor, op: "LMAOperator", overwrite: bool):
     if op.colouring is None:
         raise LfrError(1, "matrix_vector needs the operator's colouring")
-    _field(lhs, op.to_space, "lhs", op.matrix.dtype)
-    _field(x, op.from_space, "x", op.matrix.dtype)
+    _field(x, op.from_space, "x", matrix.dtype)
     plan = op.to_space.plan(op.colouring, 0)
     ctx = op.ctx
     ctx.sync_stream()
-    check(lib().lfr_matrix_vector(ctx.h, _prec(lhs), _P(lhs.data_ptr()), _P(x.data_ptr()),
-                                  _P(op.matrix.data_ptr()), op.to_space.h, op.from_space.h,
-                                  plan.h, int(overwrite)), ctx.h)
+    check(lib().lfr_matrix_vector(ctx.h, _prec(matrix), lhs.data_ptr(), x.data_ptr(), matrix.data_ptr(),
+                                  op.to_space.h, op.from_space.h, plan.h, int(overwrite)), ctx.h)
+
+
+def _dg_matrix_vector(lhs: torch.Tensor, x: torch.Tensor, matrix: torch.Tensor, op: "LMAOperator"):
+    _field(x, op.from_space, "x", matrix.dtype)
+    ctx = op.ctx
+    ctx.sync_stream()
+    check(lib().lfr_dg_matrix_vector(ctx.h, _prec(matrix), lhs.data_ptr(), x.data_ptr(), matrix.data_ptr(),
+                                     op.to_space.h, op.from_space.h), ctx.h)
+
+
+def _transpose_matrix_vector(lhs: torch.Tensor, x: torch.Tensor, matrix: torch.Tensor, op: "LMAOperator",
+                             colouring: Colouring | None, overwrite: bool):
+    if colouring is None:
+        raise LfrError(1, "transpose_matrix_vector needs a colouring of lhs' space")
+    lsp, xsp = op.from_space, op.to_space
+    _field(x, xsp, "x", matrix.dtype)
+    plan = lsp.plan(colouring, 1)
+    ctx = op.ctx
+    ctx.sync_stream()
+    check(lib().lfr_transpose_matrix_vector(ctx.h, _prec(matrix), lhs.data_ptr(), x.data_ptr(), matrix.data_ptr(),
+                                            lsp.h, xsp.h, plan.h, int(overwrite)), ctx.h)
+
+
+def matrix_vector(lhs: torch.Tensor, x: torch.Tensor, op: LMAOperator, overwrite: bool = False):
+    """lhs += M x (GH_INC, colour order); overwrite=True gives lhs = M x."""
+    _field(lhs, op.to_space, "lhs", op.matrix.dtype)
+    _matrix_vector(lhs, x, op.matrix, op, overwrite)
     return lhs
 
 
@@ -265,12 +299,7 @@ def matrix_vector_ndata(lhs: torch.Tensor, x: torch.Tensor, op: LMAOperator, ove
 def dg_matrix_vector(lhs: torch.Tensor, x: torch.Tensor, op: LMAOperator):
     """lhs = M x on a discontinuous output space."""
     _field(lhs, op.to_space, "lhs", op.matrix.dtype)
-    _field(x, op.from_space, "x", op.matrix.dtype)
-    ctx = op.ctx
-    ctx.sync_stream()
-    check(lib().lfr_dg_matrix_vector(ctx.h, _prec(lhs), _P(lhs.data_ptr()), _P(x.data_ptr()),
-                                     _P(op.matrix.data_ptr()), op.to_space.h, op.from_space.h),
-          ctx.h)
+    _dg_matrix_vector(lhs, x, op.matrix, op)
     return lhs
 
 
@@ -294,18 +323,8 @@ def transpose_matrix_vector(lhs: torch.Tensor, x: torch.Tensor, op: LMAOperator,
     same LMAOperator that maps from_space -> to_space in ``matrix_vector``
     is applied transposed here (the adjoint).
     """
-    col = colouring or op.colouring
-    if col is None:
-        raise LfrError(1, "transpose_matrix_vector needs a colouring of lhs' space")
-    lsp, xsp = op.from_space, op.to_space
-    _field(lhs, lsp, "lhs", op.matrix.dtype)
-    _field(x, xsp, "x", op.matrix.dtype)
-    plan = lsp.plan(col, 1)
-    ctx = op.ctx
-    ctx.sync_stream()
-    check(lib().lfr_transpose_matrix_vector(ctx.h, _prec(lhs), _P(lhs.data_ptr()),
-                                            _P(x.data_ptr()), _P(op.matrix.data_ptr()),
-                                            lsp.h, xsp.h, plan.h, int(overwrite)), ctx.h)
+    _field(lhs, op.from_space, "lhs", op.matrix.dtype)
+    _transpose_matrix_vector(lhs, x, op.matrix, op, colouring or op.colouring, overwrite)
     return lhs
 
 

@@ -30,7 +30,7 @@ import math
 import torch
 
 from . import api
-from ._ffi import LfrError, check, lib
+from ._ffi import check, lib
 
 
 def _zeros(space: "api.Space", dtype):
@@ -40,55 +40,33 @@ def _zeros(space: "api.Space", dtype):
 # The three kernels of an apply and its backward, called with the operator's
 # spaces and another matrix.  In a training step these calls run right after a
 # hand-over between the program's and the engine's thread, where every Python
-# statement costs several times what it costs in a loop: inputs are checked as
-# the api functions check them, buffers made here are not checked again, and
-# the stream is looked up once a backward.
+# statement costs several times what it costs in a loop: buffers made here are
+# not checked again.
 
 def _apply(M: torch.Tensor, x: torch.Tensor, op: "api.LMAOperator") -> torch.Tensor:
     op.check_matrix(M)
-    to, fr = op.to_space, op.from_space
-    discontinuous = to.fs.is_discontinuous
-    if not discontinuous and op.colouring is None:
-        raise LfrError(1, "matrix_vector needs the operator's colouring")
-    dt = M.dtype
-    p = api._prec(M)
-    api._field(x, fr, "x", dt)
-    y = torch.empty(to.undf, dtype=dt, device=M.device)
-    ctx = to.ctx
-    ctx.sync_stream()
-    if discontinuous:
-        check(lib().lfr_dg_matrix_vector(ctx.h, p, y.data_ptr(), x.data_ptr(), M.data_ptr(), to.h, fr.h), ctx.h)
+    y = torch.empty(op.to_space.undf, dtype=M.dtype, device=M.device)
+    if op.to_space.fs.is_discontinuous:
+        api._dg_matrix_vector(y, x, M, op)
     else:
-        check(lib().lfr_matrix_vector(ctx.h, p, y.data_ptr(), x.data_ptr(), M.data_ptr(), to.h, fr.h,
-                                      to.plan(op.colouring, 0).h, 1), ctx.h)
+        api._matrix_vector(y, x, M, op, True)
     return y
 
 
-def _apply_t(M: torch.Tensor, p: torch.Tensor, op: "api.LMAOperator", queued: bool = False) -> torch.Tensor:
+def _apply_t(M: torch.Tensor, p: torch.Tensor, op: "api.LMAOperator") -> torch.Tensor:
     op.check_matrix(M)
-    if op.colouring is None:
-        raise LfrError(1, "transpose_matrix_vector needs a colouring of lhs' space")
-    lsp, xsp = op.from_space, op.to_space
-    dt = M.dtype
-    prec = api._prec(M)
-    api._field(p, xsp, "x", dt)
-    b = torch.empty(lsp.undf, dtype=dt, device=M.device)
-    ctx = xsp.ctx
-    if not queued:
-        ctx.sync_stream()
-    check(lib().lfr_transpose_matrix_vector(ctx.h, prec, b.data_ptr(), p.data_ptr(), M.data_ptr(), lsp.h, xsp.h,
-                                            lsp.plan(op.colouring, 1).h, 1), ctx.h)
+    b = torch.empty(op.from_space.undf, dtype=M.dtype, device=M.device)
+    api._transpose_matrix_vector(b, p, M, op, op.colouring, True)
     return b
 
 
-def _outer(ybar: torch.Tensor, x: torch.Tensor, op: "api.LMAOperator", out=None, alpha=1.0, queued: bool = False):
+def _outer(ybar: torch.Tensor, x: torch.Tensor, op: "api.LMAOperator", out=None, alpha=1.0):
     """Mbar (+)= alpha * ybar (x) x, per cell-layer (lfr_lma_outer)."""
     acc = out is not None
     if out is None:
         out = torch.empty_like(op.matrix)
     ctx = op.ctx
-    if not queued:
-        ctx.sync_stream()
+    ctx.sync_stream()
     check(lib().lfr_lma_outer(ctx.h, api._prec(out), out.data_ptr(), ybar.data_ptr(), x.data_ptr(), op.to_space.h,
                               op.from_space.h, float(alpha), int(acc)), ctx.h)
     return out
@@ -108,7 +86,7 @@ class _LMAApply(torch.autograd.Function):
         ybar = ybar.contiguous()
         want_m, want_x, _ = ctx.needs_input_grad
         xbar = _apply_t(M, ybar, op) if want_x else None
-        Mbar = _outer(ybar, x, op, queued=want_x) if want_m else None
+        Mbar = _outer(ybar, x, op) if want_m else None
         return Mbar, xbar, None
 
 
@@ -126,7 +104,7 @@ class _LMAApplyT(torch.autograd.Function):
         bbar = bbar.contiguous()
         want_m, want_p, _ = ctx.needs_input_grad
         pbar = _apply(M, bbar, op) if want_p else None
-        Mbar = _outer(p, bbar, op, queued=want_p) if want_m else None
+        Mbar = _outer(p, bbar, op) if want_m else None
         return Mbar, pbar, None
 
 
