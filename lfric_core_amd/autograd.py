@@ -64,7 +64,7 @@ def _outer(ybar: torch.Tensor, x: torch.Tensor, op: "api.LMAOperator", out=None,
     """Mbar (+)= alpha * ybar (x) x, per cell-layer (lfr_lma_outer)."""
     acc = out is not None
     if out is None:
-        out = torch.empty_like(op.matrix)
+        out = torch.empty(op.matrix.shape, dtype=ybar.dtype, device=ybar.device)
     ctx = op.ctx
     ctx.sync_stream()
     check(lib().lfr_lma_outer(ctx.h, api._prec(out), out.data_ptr(), ybar.data_ptr(), x.data_ptr(), op.to_space.h,

@@ -70,3 +70,16 @@ def test_every_launch_sets_its_stream(rec, transpose, want, discontinuous):
     torch.autograd.grad(y, [t for t in (M, x) if t.requires_grad], torch.ones_like(y))
     assert len(rec.calls) == 1 + sum(want)
     assert [s for _, s, _ in rec.calls] == ["mine"] * len(rec.calls), rec.calls
+
+
+@pytest.mark.parametrize("transpose", [False, True])
+def test_matrix_gradient_has_the_matrix_dtype(rec, transpose):
+    """A matrix of another precision than the operator's own: its gradient is
+    formed in the precision of the fields that the kernel reads."""
+    op = _op(torch.float64)
+    M = op.matrix.float().requires_grad_()
+    x = torch.ones(UNDF_TO if transpose else UNDF_FROM, dtype=M.dtype)
+    y = (autograd.lma_apply_transpose if transpose else autograd.lma_apply)(M, x, op)
+    g, = torch.autograd.grad(y, (M,), torch.ones_like(y))
+    assert g.dtype == torch.float32
+    assert [p for _, _, p in rec.calls] == [4, 4]
