@@ -11,8 +11,9 @@
 // inv*c and inv*(x - a*d') exactly as written there.
 //
 // FP32 columns of 70 rows (W3 at 70 layers) have kernels that load a whole
-// column up front (k_appinv_deep); every other row count and kind runs
-// k_thomas_rows, which stages its loads ahead of the recurrence.
+// column up front (k_appinv_deep); other row counts and kinds run
+// k_thomas_rows, which stages its loads ahead of the recurrence; columns taller
+// than its LDS holds take generic kernels.
 #include <algorithm>
 #include <cmath>
 #include <cstdint>
@@ -455,7 +456,10 @@ size_t rows_lds(int nrow) {
 
 // IND: row r of a column is dof ind[r] - 1 of it (clamped into the column);
 // else row r is dof r
-template <typename T, typename C, typename S, bool IND>
+// ONE: one stage holds the column (up to kRowStage rows); fetching a second
+// one all the same cost C96L10 FP64 8.7 against 6.9 µs now, and operator_tri_solve
+// C128L3 FP64 11.7 against 7.1.
+template <typename T, typename C, typename S, bool IND, bool ONE>
 __global__ void __launch_bounds__(64)
 k_thomas_rows(T* __restrict__ y, S src, const int32_t* __restrict__ map0, int ndf, int cstride,
               const int32_t* __restrict__ ind, int ncell, int nrow) {
@@ -505,12 +509,14 @@ k_thomas_rows(T* __restrict__ y, S src, const int32_t* __restrict__ map0, int nd
 #pragma unroll
     for (int it = 0; it < G; ++it) src.load_field(v.f[it], base[it], off);
   };
-  const int off0 = offset(0), off1 = offset(1);
-  int off = offset(2);
+  const int off0 = offset(0), off1 = ONE ? 0 : offset(1);
+  int off = ONE ? 0 : offset(2);
   fetch_cell(0, va);
   fetch_field(va, clamped(0, off0));
-  fetch_cell(1, vb);   // a single stage reads its last row again
-  fetch_field(vb, clamped(1, off1));
+  if constexpr (!ONE) {
+    fetch_cell(1, vb);
+    fetch_field(vb, clamped(1, off1));
+  }
   C cprev = C(0), dprev = C(0);
   // NR rows from row i0 + q0: their values are read before the chain needs them
   const auto rows = [&](int i0, int q0, auto nr) {
@@ -571,12 +577,16 @@ k_thomas_rows(T* __restrict__ y, S src, const int32_t* __restrict__ map0, int nd
     __syncthreads();
   };
   int s = 0;
-  for (; s + 2 < nst; s += 2) {
-    stage(s, va, std::true_type{});
-    stage(s + 1, vb, std::true_type{});
+  if constexpr (!ONE) {
+    for (; s + 2 < nst; s += 2) {
+      stage(s, va, std::true_type{});
+      stage(s + 1, vb, std::true_type{});
+    }
   }
   stage(s, va, std::false_type{});
-  if (s + 1 < nst) stage(s + 1, vb, std::false_type{});
+  if constexpr (!ONE) {
+    if (s + 1 < nst) stage(s + 1, vb, std::false_type{});
+  }
   // backward substitution, 8 rows' c' and d' read ahead of the chain
   if (lane < kRowCols) {
     C* cpl = scp + lane * PC;
@@ -621,12 +631,16 @@ bool launch_rows(hipStream_t s, T* y, const S& src, const lfr_space* sp, const i
   const size_t lds = rows_lds<T, C>(nrow);
   if (lds > kRowLdsMax) return false;
   const dim3 grid((unsigned)((ncell + kRowCols - 1) / kRowCols));
-  if (ind)
-    hipLaunchKernelGGL((k_thomas_rows<T, C, S, true>), grid, dim3(64), lds, s, y, src, sp->map0_d, sp->ndf,
-                       sp->col_stride, ind, ncell, nrow);
-  else
-    hipLaunchKernelGGL((k_thomas_rows<T, C, S, false>), grid, dim3(64), lds, s, y, src, sp->map0_d, sp->ndf,
-                       sp->col_stride, ind, ncell, nrow);
+  const auto go = [&](auto i, auto one) {
+    hipLaunchKernelGGL((k_thomas_rows<T, C, S, decltype(i)::value, decltype(one)::value>), grid, dim3(64), lds, s, y,
+                       src, sp->map0_d, sp->ndf, sp->col_stride, ind, ncell, nrow);
+  };
+  const auto by_height = [&](auto i) {
+    if (nrow <= kRowStage) go(i, std::true_type{});
+    else go(i, std::false_type{});
+  };
+  if (ind) by_height(std::true_type{});
+  else by_height(std::false_type{});
   return true;
 }
 
@@ -696,7 +710,8 @@ int launch_appinv(lfr_ctx* ctx, T* lhs, const T* x, const T* cm, const lfr_space
       return LFR_OK;
     }
   }
-  if (!launch_rows<C>(ctx->stream, lhs, RowsBands<T>{cm, x, nrow}, sp, ind, ncell, nrow)) {
+  const RowsBands<T> src{cm, x, nrow};
+  if (!launch_rows<C>(ctx->stream, lhs, src, sp, ind, ncell, nrow)) {
     // c', d' scratch for columns taller than k_thomas_rows holds
     int rc = lfr_work_reserve(ctx, (size_t)ncell * 2 * nrow * sizeof(C) + 4096);
     if (rc) return rc;
@@ -1708,7 +1723,8 @@ bool launch_thomas(lfr_ctx* ctx, hipStream_t s, T* y, const T* x, const T* b0, c
         return true;
       }
     }
-    return launch_rows<T>(s, y, RowsFields<T>{b2, b0, b1, x}, sp, nullptr, sp->ncell, sp->nlayers);
+    const RowsFields<T> src{b2, b0, b1, x};
+    return launch_rows<T>(s, y, src, sp, nullptr, sp->ncell, sp->nlayers);
   } else {                     // operator_tri_solve: b0 = the 2x2 local matrices
     if (sp->nlayers != 70 || sizeof(T) == 8)
       return launch_rows<T>(s, y, RowsLma<T>{b0, x, sp->nlayers, (int64_t)sp->ncell * sp->nlayers}, sp, nullptr,
