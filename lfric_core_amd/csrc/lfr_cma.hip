@@ -12,8 +12,10 @@
 //
 // FP32 columns of 70 rows (W3 at 70 layers) have kernels that load a whole
 // column up front (k_appinv_deep); other row counts and kinds run
-// k_thomas_rows, which stages its loads ahead of the recurrence; columns taller
-// than its LDS holds take generic kernels.
+// k_thomas_rows, which stages its loads ahead of the recurrence.  Beside it
+// stand k_thomas_lanes, a column a lane, for FP64 recurrences on the meshes
+// where that is faster (lanes_fit), and generic kernels for columns taller
+// than the LDS of k_thomas_rows holds.
 #include <algorithm>
 #include <cmath>
 #include <cstdint>
@@ -26,6 +28,7 @@ namespace {
 
 constexpr int kCols = 64;   // columns (lanes) per workgroup
 constexpr int kCh = 14;     // rows per LDS stage of the solution store
+constexpr int kPf = 8;      // rows of loads ahead of k_thomas_lanes' recurrence
 
 // indirection_dofmap(i) - 1, clamped into the column's rows 0..nrow-1 so that
 // no access leaves the column (lfr_cma_create validates its maps; the raw
@@ -625,6 +628,112 @@ k_thomas_rows(T* __restrict__ y, S src, const int32_t* __restrict__ map0, int nd
   }
 }
 
+// ---------------------------------------------------------------------------
+// The same solve with a column a lane: its values straight from memory kPf
+// rows ahead of the recurrence (scheduling region r holds the loads of rows
+// [r kPf, (r+1) kPf) and the recurrence of the kPf rows before them), c' in
+// LDS, d' in registers, the solution through LDS for the store.  All 64 lanes
+// run recurrences, against 16 of k_thomas_rows, which counts where a row costs
+// an FP64 division, and twice the columns fit a CU; a load of 64 columns
+// touches 64 lines, which counts once those are not in the caches.  Arithmetic
+// as k_thomas_rows.  kPf: 8 rows are whole lines of an FP64 field (tri_solve
+// C72L70 22.3 µs, 23.9 with 10 rows, 22.8 with 14).
+// ---------------------------------------------------------------------------
+constexpr int kLanesPitch = kCh + 1;   // odd pitch: conflict-free lane-strided access
+
+template <typename T, typename C, typename S, bool IND, int NROW>
+__global__ void __launch_bounds__(kCols)
+k_thomas_lanes(T* __restrict__ y, S src, const int32_t* __restrict__ map0, int ndf, const int32_t* __restrict__ ind,
+               int ncell) {
+  constexpr int NST = (NROW + kCh - 1) / kCh;
+  constexpr int PC = NROW | 1;      // odd pitch of the c' rows
+  __shared__ C scp[kCols * PC];
+  __shared__ T sx[kCols * kLanesPitch];
+  __shared__ int32_t sbase[kCols];
+  __shared__ int32_t sind[IND ? NROW : 1];   // dof offset of each row
+  const int lane = threadIdx.x;
+  const int c0 = blockIdx.x * kCols;
+  const int ncols = min(kCols, ncell - c0);
+  const int c = c0 + min(lane, ncols - 1);   // idle lanes repeat a real column
+  const int64_t base = map0[(int64_t)c * ndf];
+  sbase[lane] = (int32_t)base;
+  if (IND)
+    for (int i = lane; i < NROW; i += kCols) sind[i] = ind0(ind, i, NROW);
+  C* cp = scp + lane * PC;
+  C dp[NROW];
+  {
+    T lc[NROW][S::kCell ? S::kCell : 1], lf[NROW][S::kField];
+    C cprev = C(0), dprev = C(0);
+#pragma unroll
+    for (int t = 0; t < NROW + kPf; ++t) {
+      if (t < NROW) {
+        src.load_cell(lc[t], c, t);
+        src.load_field(lf[t], base, IND ? ind0(ind, t, NROW) : t);
+      }
+      if (t >= kPf) {
+        const int i = t - kPf;
+        T o[4];
+        src.row(lc[i], lf[i], i, o);
+        const C a = (C)o[0];
+        const C ac = a * cprev;
+        const C inv = C(1) / ((C)o[1] - ac);
+        cprev = inv * (C)o[2];
+        if (i < NROW - 1) cp[i] = cprev;
+        const C ad = a * dprev;
+        dprev = inv * ((C)o[3] - ad);
+        dp[i] = dprev;
+      }
+      if ((t + 1) % kPf == 0) __builtin_amdgcn_sched_barrier(0);
+    }
+  }
+#pragma unroll
+  for (int i = NROW - 2; i >= 0; --i) {
+    const C cd = cp[i] * dp[i + 1];
+    dp[i] = dp[i] - cd;
+  }
+#pragma unroll
+  for (int s = 0; s < NST; ++s) {
+    const int r0 = s * kCh;
+    const int nr = (NROW - r0) < kCh ? (NROW - r0) : kCh;
+    __syncthreads();
+    if (lane < ncols) {
+#pragma unroll
+      for (int q = 0; q < kCh; ++q)
+        if (r0 + q < NROW) sx[lane * kLanesPitch + q] = (T)dp[r0 + q];
+    }
+    __syncthreads();
+    for (int e = lane; e < ncols * nr; e += kCols) {
+      const int cc = e / nr;
+      const int q = e - cc * nr;
+      y[(int64_t)sbase[cc] + (IND ? sind[r0 + q] : r0 + q)] = sx[cc * kLanesPitch + q];
+    }
+  }
+}
+
+// Whether k_thomas_lanes takes FP64 recurrences of nrow rows: from the mesh
+// size on at which k_thomas_rows no longer holds all columns of 70 rows at
+// once (7 workgroups a CU), as long as k_thomas_lanes does.  µs, k_thomas_rows
+// / k_thomas_lanes, operands in cache: appinv with FP64 pivots on FP32 data
+// C64L70 18.4 / 16.8, C80L70 30.9 / 21.7, C96L20 11.5 / 7.8, C96L30 15.6 / 12.0,
+// C96L50 25.6 / 20.2, C96L70 37.9 / 27.3; tri_solve FP64 C64L70 21.7 / 21.0,
+// C72L70 30.1 / 22.3, C80L70 34.8 / 29.5, C96L70 41.9 / 65.2.  Out of cache: FP64
+// pivots C64L70 18.9 / 20.6, C72L70 20.7 / 20.7, C96L70 39.7 / 36.5, C128L70
+// 57.3 / 65.9; tri_solve C72L70 33.3 / 30.3, C80L70 38.9 / 39.7, C96L70 46.3 /
+// 69.8.  (appinv on FP64 data: C80L70 33.8 / 30.0 in cache, 36.8 / 44.7 out of
+// it: k_thomas_rows.)
+template <typename T>
+bool lanes_fit(int ncell, int nrow) {
+  constexpr int kCus = 256, kLdsCu = 160 * 1024;
+  const int lds = kCols * ((nrow | 1) * 8 + kLanesPitch * (int)sizeof(T) + 4) + nrow * 4;
+  return ncell > kCus * 7 * kRowCols && ncell <= kCus * kCols * (kLdsCu / lds);
+}
+
+template <typename T, typename C, bool IND, int NROW, typename S>
+void launch_lanes(hipStream_t s, T* y, const S& src, const lfr_space* sp, const int32_t* ind, int ncell) {
+  hipLaunchKernelGGL((k_thomas_lanes<T, C, S, IND, NROW>), dim3((unsigned)((ncell + kCols - 1) / kCols)), dim3(kCols), 0,
+                     s, y, src, sp->map0_d, sp->ndf, ind, ncell);
+}
+
 // Queue a solve; false when the columns are too tall for its LDS
 template <typename C, typename T, typename S>
 bool launch_rows(hipStream_t s, T* y, const S& src, const lfr_space* sp, const int32_t* ind, int ncell, int nrow) {
@@ -711,6 +820,20 @@ int launch_appinv(lfr_ctx* ctx, T* lhs, const T* x, const T* cm, const lfr_space
     }
   }
   const RowsBands<T> src{cm, x, nrow};
+  if constexpr (sizeof(C) > sizeof(T)) {
+    if (lanes_fit<T>(ncell, nrow)) {
+      switch (nrow) {   // the row counts of usual layer counts
+#define CASE(NR)                                                           \
+  case NR:                                                                 \
+    launch_lanes<T, C, true, NR>(ctx->stream, lhs, src, sp, ind, ncell);   \
+    LFR_CHECK_LAUNCH(ctx);                                                 \
+    return LFR_OK;
+        CASE(20) CASE(21) CASE(30) CASE(31) CASE(50) CASE(51) CASE(70) CASE(71)
+#undef CASE
+        default: break;
+      }
+    }
+  }
   if (!launch_rows<C>(ctx->stream, lhs, src, sp, ind, ncell, nrow)) {
     // c', d' scratch for columns taller than k_thomas_rows holds
     int rc = lfr_work_reserve(ctx, (size_t)ncell * 2 * nrow * sizeof(C) + 4096);
@@ -1724,6 +1847,12 @@ bool launch_thomas(lfr_ctx* ctx, hipStream_t s, T* y, const T* x, const T* b0, c
       }
     }
     const RowsFields<T> src{b2, b0, b1, x};
+    if constexpr (sizeof(T) == 8) {
+      if (sp->nlayers == 70 && lanes_fit<T>(sp->ncell, 70)) {
+        launch_lanes<T, T, false, 70>(s, y, src, sp, nullptr, sp->ncell);
+        return true;
+      }
+    }
     return launch_rows<T>(s, y, src, sp, nullptr, sp->ncell, sp->nlayers);
   } else {                     // operator_tri_solve: b0 = the 2x2 local matrices
     if (sp->nlayers != 70 || sizeof(T) == 8)

@@ -118,3 +118,29 @@ def test_appinv_any_height_bitexact(ctx, dtype, nl):
         api.columnwise_op_appinv(y, xd, op, fp64_pivots=True)
         torch.cuda.synchronize()
         np.testing.assert_array_equal(y.cpu().numpy(), ref64.astype(np.float32))
+
+
+@pytest.mark.parametrize("nl", [19, 20, 21, 30, 31, 50, 51, 70, 71])
+def test_appinv_fp64_pivots_on_large_meshes_bitexact(ctx, nl):
+    """29,400 columns (a partial wave at the end): the row counts that have the
+    column-a-lane kernel there and one that has not, a permuted indirection,
+    lhs by itself and in place of x, against the FP64 solve rounded to FP32."""
+    from lfric_core_amd import api
+    print(f"case appinv FP64 pivots C70 nl={nl}", flush=True)
+    m = cubed_sphere(70)
+    w3 = build_dofmap(m, "W3", nl)
+    st = Stream(39)
+    cm = _helmholtz_columns(st, m.ncells, nl).astype(np.float32)
+    x = st.uniform(w3.undf).astype(np.float32)
+    ind = (np.random.default_rng(7).permutation(nl) + 1).astype(np.int32)
+    ref = oracle.appinv(np.zeros(w3.undf), x.astype(np.float64), cm.astype(np.float64), w3.dofmap, ind).astype(np.float32)
+    sp = api.Space(ctx, w3)
+    op = api.CMAOperator(torch.from_numpy(cm).to(ctx.device), sp, ind)
+    xd = torch.from_numpy(x).to(ctx.device)
+    y = torch.full_like(xd, float("nan"))
+    api.columnwise_op_appinv(y, xd, op, fp64_pivots=True)
+    z = xd.clone()
+    api.columnwise_op_appinv(z, z, op, fp64_pivots=True)
+    torch.cuda.synchronize()
+    np.testing.assert_array_equal(y.cpu().numpy(), ref)
+    np.testing.assert_array_equal(z.cpu().numpy(), ref)

@@ -163,3 +163,26 @@ def test_tri_solves_of_any_height_bitexact(ctx, dtype, nl, permuted):
             api.operator_tri_solve(y, _t(x, ctx), _t(m, ctx), sp)
         torch.cuda.synchronize()
         np.testing.assert_array_equal(y.cpu().numpy(), ref)
+
+
+@pytest.mark.parametrize("permuted", [False, True])
+@pytest.mark.parametrize("nl", [70, 71])
+def test_tri_solve_fp64_large_mesh_bitexact(ctx, nl, permuted):
+    """29,400 columns: at 70 rows the column-a-lane kernel, at 71 the staged one."""
+    import dataclasses
+    from lfric_core_amd import api
+    print(f"case tri solve C70 nl={nl} permuted={permuted}", flush=True)
+    mesh = cubed_sphere(70)
+    fs = build_dofmap(mesh, "W3", nl)
+    if permuted:
+        perm = np.random.default_rng(9).permutation(mesh.ncells)
+        fs = dataclasses.replace(fs, dofmap=np.ascontiguousarray(fs.dofmap[perm]))
+    st = Stream(56)
+    sp = api.Space(ctx, fs)
+    x, t0 = st.uniform(fs.undf), 4.0 + st.uniform(fs.undf)
+    tp, tm = 0.5 * st.uniform(fs.undf), 0.5 * st.uniform(fs.undf)
+    ref = oracle.tri_solve(np.zeros(fs.undf), x, t0, tp, tm, fs.dofmap, nl)
+    y = torch.full((fs.undf,), float("nan"), dtype=torch.float64, device=ctx.device)
+    api.tri_solve(y, _t(x, ctx), _t(t0, ctx), _t(tp, ctx), _t(tm, ctx), sp)
+    torch.cuda.synchronize()
+    np.testing.assert_array_equal(y.cpu().numpy(), ref)
