@@ -154,19 +154,31 @@ void launch_bundles(hipStream_t s, int kind, const T* M, const T* x, T* y, const
                        n3, ndf_out, ndf_in, nf, overwrite, nbp);
 }
 
-template <typename T, int F>
-void launch_one(hipStream_t s, int kind, const T* M, const T* x, T* y, const int32_t* mi, const lfr::BunClass& bc,
-                int nl, int64_t n3, int ndf_out, int ndf_in, int nf, int overwrite) {
+template <typename T, int F, int UMAX>
+void launch_one_u(hipStream_t s, int kind, const T* M, const T* x, T* y, const int32_t* mi, const lfr::BunClass& bc,
+                  int nl, int64_t n3, int ndf_out, int ndf_in, int nf, int overwrite) {
   const unsigned nbp = pad8(bc.nblocks);
 #define LONE(GSV, KD, MK)                                                                                      \
-  hipLaunchKernelGGL((lfr::k_gather_one<T, F, GSV, KD, MK>), dim3(nbp), dim3(kThreads), 0, s, M, x, y, mi, bc, nl, n3, \
-                     ndf_out, ndf_in, nf, overwrite, nbp)
+  hipLaunchKernelGGL((lfr::k_gather_one<T, F, GSV, KD, MK, UMAX>), dim3(nbp), dim3(kThreads), 0, s, M, x, y, mi, bc, \
+                     nl, n3, ndf_out, ndf_in, nf, overwrite, nbp)
   if (kind == 0) {
     if (bc.gs == 0) LONE(1, 0, false); else if (bc.gs == 1) LONE(1, 0, true); else LONE(2, 0, true);
   } else {
     if (bc.gs == 0) LONE(1, 1, false); else if (bc.gs == 1) LONE(1, 1, true); else LONE(2, 1, true);
   }
 #undef LONE
+}
+
+// Up to three input dofs a cell (2: Wtheta, W2V): blocks of two, one trip, in a
+// kernel of few registers.  With four a block the two took a trip each:
+// Wtheta C96L70 FP32 28.0 against 20.4 µs now, FP64 55.4 against 39.5, 7 fields
+// C48L70 FP64 79.1 against 53.5 (four a block with a trip of two after it 22.6,
+// 50.5, 73.9; one a block 24.7, 46.3, 63.4).
+template <typename T, int F>
+void launch_one(hipStream_t s, int kind, const T* M, const T* x, T* y, const int32_t* mi, const lfr::BunClass& bc,
+                int nl, int64_t n3, int ndf_out, int ndf_in, int nf, int overwrite) {
+  if (ndf_in < 4) launch_one_u<T, F, 2>(s, kind, M, x, y, mi, bc, nl, n3, ndf_out, ndf_in, nf, overwrite);
+  else launch_one_u<T, F, 4>(s, kind, M, x, y, mi, bc, nl, n3, ndf_out, ndf_in, nf, overwrite);
 }
 
 // Bundles of the first class a chunk of the interleaved launch takes (4 and

@@ -504,7 +504,7 @@ struct BunClasses {
   unsigned nchunk;
 };
 
-template <typename T, int R, int F, int GS, int KIND, bool MASK>
+template <typename T, int R, int F, int GS, int KIND, bool MASK, int UMAX = 4>
 __device__ __forceinline__ void gather_bun_body(const T* __restrict__ M, const T* __restrict__ x, T* __restrict__ y,
                                                 const int32_t* __restrict__ map_in, const BunClass& bc, unsigned blk,
                                                 int nl, int64_t n3, int ndf_out, int ndf_in, int nf, int overwrite) {
@@ -615,7 +615,7 @@ __device__ __forceinline__ void gather_bun_body(const T* __restrict__ M, const T
     };
     // loads in flight against registers: two input dofs at a time where two
     // entries' rows of FP64 pairs would not leave two waves a SIMD
-    constexpr int U = GS * R > 4 ? 2 : 4;
+    constexpr int U = GS * R > 4 && UMAX > 2 ? 2 : UMAX;
     int j = 0;
     for (; j + U <= ndf_in; j += U) dofs(j, std::integral_constant<int, U>{});
     for (; j < ndf_in; ++j) dofs(j, std::integral_constant<int, 1>{});
@@ -978,13 +978,14 @@ k_gather_bun(const T* __restrict__ M, const T* __restrict__ x, T* __restrict__ y
   }
 }
 
-// One class with one column a bundle (no rows to share an operand value)
-template <typename T, int F, int GS, int KIND, bool MASK>
+// One class with one column a bundle (no rows to share an operand value);
+// blocks of UMAX input dofs
+template <typename T, int F, int GS, int KIND, bool MASK, int UMAX>
 __global__ void __launch_bounds__(kThreads)
 k_gather_one(const T* __restrict__ M, const T* __restrict__ x, T* __restrict__ y, const int32_t* __restrict__ map_in,
              BunClass bc, int nl, int64_t n3, int ndf_out, int ndf_in, int nf, int overwrite, unsigned nb_pad) {
-  gather_bun_body<T, 1, F, GS, KIND, MASK>(M, x, y, map_in, bc, lfr_xcd_block(blockIdx.x, nb_pad), nl, n3, ndf_out,
-                                           ndf_in, nf, overwrite);
+  gather_bun_body<T, 1, F, GS, KIND, MASK, UMAX>(M, x, y, map_in, bc, lfr_xcd_block(blockIdx.x, nb_pad), nl, n3,
+                                                 ndf_out, ndf_in, nf, overwrite);
 }
 
 // ---------------------------------------------------------------------------

@@ -153,3 +153,46 @@ def test_quads_across_bundles_bitexact(ctx, dtype, nl):
                 ref = oracle.invoke_coloured(kind, col, nl, np.zeros(fs.undf, dtype), np.ascontiguousarray(X[:, r]), M,
                                              fs.dofmap, fs.dofmap)
                 np.testing.assert_array_equal(y[:, r].cpu().numpy(), ref)
+
+
+def _check_against_oracle(ctx, label, op, tr, fields, st):
+    """matrix_vector (tr: transpose_matrix_vector) on 1 (None: the single-field
+    call) to several fields, increment and overwrite, bit for bit."""
+    from lfric_core_amd import api
+    lsp, xsp = (op.from_space, op.to_space) if tr else (op.to_space, op.from_space)
+    nl, dtype = lsp.fs.nlayers, np.float32 if op.matrix.dtype == torch.float32 else np.float64
+    M = op.matrix.cpu().numpy()
+    for nd in fields:
+        print(f"case {label} transpose={tr} nl={nl} nd={nd} {dtype.__name__}", flush=True)
+        n = nd or 1
+        X = st.uniform(xsp.undf * n).reshape(xsp.undf, n).astype(dtype)
+        Y0 = st.uniform(lsp.undf * n).reshape(lsp.undf, n).astype(dtype)
+        for over in (False, True):
+            y = _t(np.full_like(Y0, np.nan) if over else Y0, ctx)
+            if nd is None:
+                call = api.transpose_matrix_vector if tr else api.matrix_vector
+                call(y.view(-1), _t(X, ctx).view(-1), op, overwrite=over)
+            else:
+                api.matrix_vector_ndata(y, _t(X, ctx), op, overwrite=over, transpose=tr)
+            y = y.cpu().numpy()
+            for r in sorted({0, n // 2, n - 1}):
+                start = np.zeros(lsp.undf, dtype) if over else np.ascontiguousarray(Y0[:, r])
+                ref = oracle.invoke_coloured(int(tr), op.colouring, nl, start, np.ascontiguousarray(X[:, r]), M,
+                                             lsp.fs.dofmap, xsp.fs.dofmap)
+                np.testing.assert_array_equal(y[:, r], ref)
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("nl", [1, 2, 5])
+@pytest.mark.parametrize("to,frm", [("WTHETA", "WTHETA"), ("W2V", "W2V"), ("W2", "WTHETA"), ("W2", "W3"),
+                                    ("WTHETA", "W3")])
+def test_few_input_dofs_bitexact(ctx, dtype, nl, to, frm):
+    """One and two input dofs a cell: less than a block of the gather."""
+    from lfric_core_amd import api
+    m, col, fs, sp = _setup(ctx, 5, nl, 0, {to, frm})
+    st = Stream(35)
+    M = normal_lma(st, m.ncells * nl, fs[to].ndf, fs[frm].ndf).astype(dtype)
+    op = api.LMAOperator(_t(M, ctx), sp[to], sp[frm], col)
+    for tr in (False, True):
+        if not sp[frm if tr else to].fs.is_discontinuous:
+            _check_against_oracle(ctx, f"{to}<-{frm}", op, tr, (None, 1, 2, 3, 4, 6, 7), st)
