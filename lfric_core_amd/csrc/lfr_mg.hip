@@ -36,6 +36,7 @@
 #include <cstdlib>
 #include <cstring>
 #include <cmath>
+#include <type_traits>
 #include <vector>
 
 #include "lfr_internal.h"
@@ -532,26 +533,27 @@ __global__ void __launch_bounds__(256) k_mg_smooth_nl(T* __restrict__ xo, const 
 // (x one layer up, b, the four neighbours, the bands) in flight while the
 // chunk before it is summed, d' in LDS ([layer][lane], so xo is written once),
 // the backward sweep's cp a chunk of CB layers ahead.  KX keeps x in LDS too
-// instead of reading it again in the backward sweep.  One wave a workgroup: the
-// LDS of the columns, not registers, sets how many are in flight (8 waves a CU
-// at 70 layers FP32), and the chunks in flight make up for it.  Same operations
+// instead of reading it again in the backward sweep.  Each wave has LDS of its
+// own; that of the columns, not registers, sets how many are in flight (8 waves
+// a CU at 70 layers FP32), and the chunks in flight make up for it.  Same operations
 // and order as k_mg_smooth_nl.  Against a sweep that loaded layer by layer and
 // kept d' in xo (one solve of one V-cycle, conversions as now): C96L60 FP32
 // 1790 -> 970 µs, C72L85 FP64 2870 -> 1821, C48L33 FP32 350 -> 164, C40L100
 // FP64 one field 1810 -> 800.  At 70 layers k_mg_smooth_nl stays: C96L70 FP32
 // 1018 against 1212 µs, FP64 2372 against 2555 (its registers hold twice the
 // columns that LDS does).
-template <typename T, bool KX>
-__global__ void __launch_bounds__(64) k_mg_smooth_rt(T* __restrict__ xo, const T* __restrict__ xi,
+template <typename T, bool KX, int BS>
+__global__ void __launch_bounds__(BS) k_mg_smooth_rt(T* __restrict__ xo, const T* __restrict__ xi,
                                                      const T* __restrict__ b, const Band4<T>* __restrict__ adui,
                                                      const T* __restrict__ cp, const int32_t* __restrict__ nb,
                                                      int ncell, int nl, int lgR, T sigma, T omega, unsigned nb_pad) {
   constexpr int CH = 4, CB = 8;
   extern __shared__ double smem_mg[];
-  T* sd = reinterpret_cast<T*>(smem_mg) + threadIdx.x;
+  T* sd = reinterpret_cast<T*>(smem_mg) + (threadIdx.x & 63);
+  if (BS > 64) sd += (threadIdx.x >> 6) * ((KX ? 2 : 1) * nl * 64);
   T* sx = sd + nl * 64;   // KX only
   const int R = 1 << lgR;
-  const int64_t t0 = (int64_t)lfr_xcd_block(blockIdx.x, nb_pad) * 64 + threadIdx.x;
+  const int64_t t0 = (int64_t)lfr_xcd_block(blockIdx.x, nb_pad) * BS + threadIdx.x;
   const int64_t plane = (int64_t)ncell * R;
   if (t0 >= plane) return;   // no barrier below: a lane uses its own LDS column only
   const int64_t t = t0;
@@ -670,6 +672,28 @@ int lg2(int v) {
   return l;
 }
 
+// k_mg_smooth_rt keeps x beside d' in LDS while that still leaves 8 waves a CU
+// (µs a V-cycle with and without: C48L33 FP32 175 / 178, C12L10 FP64 87 / 90; at
+// 30 KB C96L60 FP32 1151 / 1115)
+template <typename T>
+bool smooth_rt_kx(int nl) {
+  return 2 * (size_t)nl * 64 * sizeof(T) <= 20 * 1024;
+}
+
+template <typename T>
+size_t smooth_rt_lds(int nl) {   // bytes a wave
+  return (smooth_rt_kx<T>(nl) ? 2 : 1) * (size_t)nl * 64 * sizeof(T);
+}
+
+// Largest workgroup of the smoother: 256, or as many waves as 64 KiB of LDS hold
+template <typename T>
+int smooth_max_block(int nl) {
+  if (nl == 70) return 256;
+  int bs = 256;
+  while (bs > 64 && (size_t)(bs / 64) * smooth_rt_lds<T>(nl) > 64 * 1024) bs /= 2;
+  return bs;
+}
+
 template <typename T>
 void launch_smooth(hipStream_t s, lfr_mg* mg, lfr_mg_level& L, T* xo, const T* xi) {
   const int bs = L.block_smooth;
@@ -698,19 +722,20 @@ void launch_smooth(hipStream_t s, lfr_mg* mg, lfr_mg_level& L, T* xo, const T* x
                          lg2(mg->nrhs), (T)L.sigma, (T)mg->omega, nbp);
     return;
   }
-  // x beside d' in LDS while that still leaves 8 waves a CU (µs a V-cycle with
-  // and without: C48L33 FP32 175 / 178, C12L10 FP64 87 / 90; at 30 KB C96L60
-  // FP32 1151 / 1115)
-  const size_t lds = (size_t)mg->nl * 64 * sizeof(T);
-  const unsigned nbp = ((unsigned)((n + 63) / 64) + 7u) & ~7u;
-  if (2 * lds <= 20 * 1024)
-    hipLaunchKernelGGL((k_mg_smooth_rt<T, true>), dim3(nbp), dim3(64), 2 * lds, s, xo, xi, (const T*)L.b_d,
-                       (const Band4<T>*)L.adui_d, (const T*)L.cp_d, L.cell_next_d, L.ncell, mg->nl, lg2(mg->nrhs),
-                       (T)L.sigma, (T)mg->omega, nbp);
-  else
-    hipLaunchKernelGGL((k_mg_smooth_rt<T, false>), dim3(nbp), dim3(64), lds, s, xo, xi, (const T*)L.b_d,
-                       (const Band4<T>*)L.adui_d, (const T*)L.cp_d, L.cell_next_d, L.ncell, mg->nl, lg2(mg->nrhs),
-                       (T)L.sigma, (T)mg->omega, nbp);
+  const auto go = [&](auto kx, auto block) {
+    constexpr int BS = decltype(block)::value;
+    const unsigned nbp = ((unsigned)((n + BS - 1) / BS) + 7u) & ~7u;
+    hipLaunchKernelGGL((k_mg_smooth_rt<T, decltype(kx)::value, BS>), dim3(nbp), dim3(BS),
+                       BS / 64 * smooth_rt_lds<T>(mg->nl), s, xo, xi, (const T*)L.b_d, (const Band4<T>*)L.adui_d,
+                       (const T*)L.cp_d, L.cell_next_d, L.ncell, mg->nl, lg2(mg->nrhs), (T)L.sigma, (T)mg->omega, nbp);
+  };
+  const auto by_block = [&](auto kx) {
+    if (bs == 256) go(kx, std::integral_constant<int, 256>{});
+    else if (bs == 128) go(kx, std::integral_constant<int, 128>{});
+    else go(kx, std::integral_constant<int, 64>{});
+  };
+  if (smooth_rt_kx<T>(mg->nl)) by_block(std::true_type{});
+  else by_block(std::false_type{});
 }
 
 // two sweeps: x -> t -> x
@@ -778,12 +803,18 @@ void mg_free(lfr_mg* mg) {
 // Pick the workgroup size of the smoother (the dominant kernel) for each
 // level through the autotuner (one sweep per candidate size, identical
 // results), keyed by the level's shape so that levels of the same size and
-// later hierarchies reuse the choice.
+// later hierarchies reuse the choice.  Tall columns whose LDS holds one wave
+// only leave nothing to choose.
 template <typename T>
 int autotune(lfr_mg* mg) {
   lfr_ctx* ctx = mg->ctx;
   const int cand[3] = {64, 128, 256};   // launch bound of the smoother is 256
+  int n = 1;
+  while (n < 3 && cand[n] <= smooth_max_block<T>(mg->nl)) ++n;
   for (auto& L : mg->lev) {
+    L.block_smooth = cand[n - 1];
+    L.block_other = 256;
+    if (n == 1) continue;
     char key[128];
     snprintf(key, sizeof key, "mg smooth prec=%d nl=%d ncell=%d rhs=%d", (int)sizeof(T), mg->nl, L.ncell,
              mg->nrhs);
@@ -792,8 +823,7 @@ int autotune(lfr_mg* mg) {
       launch_smooth<T>(ctx->stream, mg, L, (T*)L.t_d, (const T*)L.x_d);
       return hipGetLastError() == hipSuccess ? LFR_OK : LFR_ERR_HIP;
     };
-    L.block_smooth = cand[lfr_tune_pick(ctx, key, 3, 2, run)];
-    L.block_other = 256;   // (other layer counts smooth with one wave a workgroup)
+    L.block_smooth = cand[lfr_tune_pick(ctx, key, n, n - 1, run)];
   }
   return LFR_OK;
 }

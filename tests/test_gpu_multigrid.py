@@ -115,3 +115,33 @@ def test_bad_arguments(ctx):
     H.levels[1].children[0, 0] = H.levels[1].children[0, 1]
     with pytest.raises(LfrError):
         Multigrid(ctx, H, prec=8, nrhs=1)
+
+
+@pytest.mark.parametrize("prec,nl,sizes", [(4, 10, (64, 128, 256)), (8, 9, (64, 128, 256)), (8, 33, (64, 128)),
+                                           (4, 100, (64, 128)), (8, 100, (64,)), (8, 128, (64,)),
+                                           (4, 70, (64, 128, 256))])
+def test_smoother_runs_at_the_chosen_workgroup_size(ctx, monkeypatch, prec, nl, sizes):
+    """Every stored choice is the size that the smoother reports and runs at,
+    bit for bit; sizes whose columns' LDS is past 64 KiB are not among them."""
+    H = build_hierarchy((6, 3), nlayers=nl)
+    keys = [f"mg smooth prec={prec} nl={nl} ncell={L.ncell} rhs=2" for L in H.levels]
+    for c, size in enumerate(sizes):
+        print(f"mg smoother prec={prec} nl={nl} size={size}", flush=True)
+        ctx.tune_clear()
+        for k in keys:
+            ctx.tune_set(k, c)
+        mg = Multigrid(ctx, H, prec=prec, nrhs=2)
+        assert mg.block_sizes == [size, size]
+        mg.close()
+        x, res, xo, reso = _run(ctx, H, prec, nrhs=2, ncycles=1)
+        np.testing.assert_array_equal(x, xo)
+    ctx.tune_clear()
+    mg = Multigrid(ctx, H, prec=prec, nrhs=2)   # timed; one size leaves nothing to time
+    assert all(b in sizes for b in mg.block_sizes)
+    assert len(ctx.tune_entries()) == (2 if len(sizes) > 1 else 0)
+    mg.close()
+    ctx.tune_clear()
+    monkeypatch.setenv("LFR_TUNE", "0")
+    mg = Multigrid(ctx, H, prec=prec, nrhs=2)
+    assert mg.block_sizes == [sizes[-1]] * 2
+    mg.close()
