@@ -1855,39 +1855,39 @@ bool launch_thomas(lfr_ctx* ctx, hipStream_t s, T* y, const T* x, const T* b0, c
     }
     return launch_rows<T>(s, y, src, sp, nullptr, sp->ncell, sp->nlayers);
   } else {                     // operator_tri_solve: b0 = the 2x2 local matrices
-    if (sp->nlayers != 70 || sizeof(T) == 8)
-      return launch_rows<T>(s, y, RowsLma<T>{b0, x, sp->nlayers, (int64_t)sp->ncell * sp->nlayers}, sp, nullptr,
-                            sp->ncell, sp->nlayers + 1);
     if constexpr (sizeof(T) == 4) {
-      // result-identical variants (columns a wave x rows a stage, the staged
-      // kernel) chosen by the autotuner on the first call of a shape
-      const int ncell = sp->ncell;
-      const auto launch = [&](int c) -> int {
-        switch (c) {
-          case 0:
-            hipLaunchKernelGGL((k_optri_deep<71, 12, 16>), dim3((ncell + 15) / 16), dim3(kCols), 0, s, y, x, b0,
-                               sp->map0_d, sp->ndf, ncell, sp->col_stride);
-            break;
-          case 1:
-            hipLaunchKernelGGL((k_optri_deep<71, 8, 32>), dim3((ncell + 31) / 32), dim3(kCols), 0, s, y, x, b0,
-                               sp->map0_d, sp->ndf, ncell, sp->col_stride);
-            break;
-          default:
-            hipLaunchKernelGGL((k_optri_staged<T, 71, kCh>), dim3(nb), dim3(kCols), 0, s, y, x, b0, sp->map0_d,
-                               sp->ndf, ncell, sp->nlayers);
-        }
-        return hipGetLastError() == hipSuccess ? LFR_OK : LFR_ERR_HIP;
-      };
-      char key[96];
-      snprintf(key, sizeof key, "operator_tri_solve f32 nl=70 ncell=%d", ncell);
-      // untuned default: 32 columns a wave while that still gives few
-      // enough waves for one pass over the chip, else 16
-      const int dflt = (ncell + 31) / 32 <= 2048 ? 1 : 0;
-      const int c = ctx ? lfr_tune_pick(ctx, key, 3, dflt, launch) : dflt;
-      (void)launch(c);
-      return true;
+      if (sp->nlayers == 70) {
+        // result-identical variants (columns a wave x rows a stage, the staged
+        // kernel) chosen by the autotuner on the first call of a shape
+        const int ncell = sp->ncell;
+        const auto launch = [&](int c) -> int {
+          switch (c) {
+            case 0:
+              hipLaunchKernelGGL((k_optri_deep<71, 12, 16>), dim3((ncell + 15) / 16), dim3(kCols), 0, s, y, x, b0,
+                                 sp->map0_d, sp->ndf, ncell, sp->col_stride);
+              break;
+            case 1:
+              hipLaunchKernelGGL((k_optri_deep<71, 8, 32>), dim3((ncell + 31) / 32), dim3(kCols), 0, s, y, x, b0,
+                                 sp->map0_d, sp->ndf, ncell, sp->col_stride);
+              break;
+            default:
+              hipLaunchKernelGGL((k_optri_staged<T, 71, kCh>), dim3(nb), dim3(kCols), 0, s, y, x, b0, sp->map0_d,
+                                 sp->ndf, ncell, sp->nlayers);
+          }
+          return hipGetLastError() == hipSuccess ? LFR_OK : LFR_ERR_HIP;
+        };
+        char key[96];
+        snprintf(key, sizeof key, "operator_tri_solve f32 nl=70 ncell=%d", ncell);
+        // untuned default: 32 columns a wave while that still gives few
+        // enough waves for one pass over the chip, else 16
+        const int dflt = (ncell + 31) / 32 <= 2048 ? 1 : 0;
+        const int c = ctx ? lfr_tune_pick(ctx, key, 3, dflt, launch) : dflt;
+        (void)launch(c);
+        return true;
+      }
     }
-    return false;
+    return launch_rows<T>(s, y, RowsLma<T>{b0, x, sp->nlayers, (int64_t)sp->ncell * sp->nlayers}, sp, nullptr,
+                          sp->ncell, sp->nlayers + 1);
   }
 }
 

@@ -128,15 +128,19 @@ void launch_gather_shape(hipStream_t s, int kind, unsigned nb, const T* M, const
     launch_gather_t<T, NDF_IN, 0, 2>(s, kind, nb, M, x, y, mi, c, nl, n3, ndf_out, ndf_in, overwrite);
 }
 
+// Numbers of input dofs with gathers of their own; the rest take run_bundles
+bool gather_has(int ndf_in) { return ndf_in == 1 || ndf_in == 6 || ndf_in == 8; }
+
+// False for a number of input dofs that gather_has does not name
 template <typename T>
-void launch_gather_any(hipStream_t s, int kind, unsigned nb, const T* M, const T* x, T* y,
+bool launch_gather_any(hipStream_t s, int kind, unsigned nb, const T* M, const T* x, T* y,
                        const int32_t* mi, const lfr_plan_class& c, int nl, int64_t n3, int ndf_out,
                        int ndf_in, int overwrite) {
   switch (ndf_in) {
-    case 1: launch_gather_shape<T, 1>(s, kind, nb, M, x, y, mi, c, nl, n3, ndf_out, ndf_in, overwrite); break;
-    case 6: launch_gather_shape<T, 6>(s, kind, nb, M, x, y, mi, c, nl, n3, ndf_out, ndf_in, overwrite); break;
-    case 8: launch_gather_shape<T, 8>(s, kind, nb, M, x, y, mi, c, nl, n3, ndf_out, ndf_in, overwrite); break;
-    default: break;   // run_bundles
+    case 1: launch_gather_shape<T, 1>(s, kind, nb, M, x, y, mi, c, nl, n3, ndf_out, ndf_in, overwrite); return true;
+    case 6: launch_gather_shape<T, 6>(s, kind, nb, M, x, y, mi, c, nl, n3, ndf_out, ndf_in, overwrite); return true;
+    case 8: launch_gather_shape<T, 8>(s, kind, nb, M, x, y, mi, c, nl, n3, ndf_out, ndf_in, overwrite); return true;
+    default: return false;
   }
 }
 
@@ -354,7 +358,7 @@ int run_gather(lfr_ctx* ctx, const lfr_plan* plan, int kind, const T* M, const T
     LFR_CHECK_LAUNCH(ctx);
     return LFR_OK;
   }
-  if (!pk && in->ndf != 1 && in->ndf != 6 && in->ndf != 8)
+  if (!pk && !gather_has(in->ndf))
     return run_bundles<T>(ctx, plan, kind, M, x, y, in, ndf_out, n3, 1, overwrite);
   for (size_t ci = 0; ci < plan->classes.size(); ++ci) {
     const auto& c = plan->classes[ci];
@@ -391,8 +395,8 @@ int run_gather(lfr_ctx* ctx, const lfr_plan* plan, int kind, const T* M, const T
     if (c.gsize != 1 && c.gsize != 2)
       return lfr_set_error(ctx, LFR_ERR_ARG, "plan class with %d entries per cell unsupported",
                            c.gsize);
-    launch_gather_any<T>(ctx->stream, kind, nb, M, x, y, in->map0_d, c, nl, n3, ndf_out, in->ndf,
-                         overwrite);
+    if (!launch_gather_any<T>(ctx->stream, kind, nb, M, x, y, in->map0_d, c, nl, n3, ndf_out, in->ndf, overwrite))
+      return lfr_set_error(ctx, LFR_ERR_ARG, "no gather for %d input dofs a cell", in->ndf);
     LFR_CHECK_LAUNCH(ctx);
   }
   return LFR_OK;
