@@ -206,12 +206,14 @@ def _limited_area(n):
 
 
 @pytest.mark.parametrize("dtype", [np.float32, np.float64])
-@pytest.mark.parametrize("space,k,nl", [("W2", 0, 4), ("W2", 0, 5), ("W0", 0, 3), ("W0", 1, 2), ("W2", 1, 2)])
-def test_few_columns_join_a_larger_class(ctx, dtype, space, k, nl):
-    """A 72 x 72 limited area: the edge's columns, which fewer cells touch, are
-    a small part of all and take the larger class's kernel with absent
-    entries; matrix_vector and its transpose, packed and not, increment and
-    overwrite, bit for bit against the oracle."""
+@pytest.mark.parametrize("space,k,nl,nclasses", [("W2", 0, 4, 2), ("W2", 0, 5, 2), ("W0", 0, 3, 1), ("W0", 1, 2, 6),
+                                                 ("W2", 1, 2, 3)])
+def test_few_columns_join_a_larger_class(ctx, dtype, space, k, nl, nclasses):
+    """A 72 x 72 limited area.  At lowest order the edge's columns, which fewer
+    cells touch, are a small part of all and take the larger class's kernel
+    with absent entries (1 class for W0's 3, 2 for W2's 3); at order 1 no class
+    is small enough and none joins (6 and 3).  matrix_vector and its transpose,
+    packed and not, increment and overwrite, bit for bit against the oracle."""
     from lfric_core_amd import api
     print(f"case absent entries {space} k={k} nl={nl} {dtype.__name__}", flush=True)
     m = _limited_area(72)
@@ -223,6 +225,7 @@ def test_few_columns_join_a_larger_class(ctx, dtype, space, k, nl):
     dev = lambda a: torch.from_numpy(a.copy()).to(ctx.device)
     op = api.LMAOperator(dev(M), sp, sp, col)
     for kind, call in ((0, api.matrix_vector), (1, api.transpose_matrix_vector)):
+        assert sp.plan(col, kind).info()["nclasses"] == nclasses
         for over in (False, True):
             start = np.zeros_like(y0) if over else y0.copy()
             ref = oracle.invoke_coloured(kind, col, nl, start, x, M, fs.dofmap, fs.dofmap)

@@ -250,3 +250,39 @@ def test_cg_x_has_every_step_up_to_the_stop(ctx, edge, nlayers, diag):
             assert st.iterations == it and bool(st.converged) == by_tol
             assert np.linalg.norm(x.cpu().numpy() - xo) <= 1e-11 * np.linalg.norm(xo)
         ratio = rn / r0
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("packed", [False, True])
+def test_cg_on_a_limited_area(ctx, dtype, packed):
+    """A 40 x 40 limited area, whose edge faces have joined the class of the
+    inner ones, so that the apply with the fused dot product is the unified
+    gather with absent entries: 15 fixed iterations against the oracle, which
+    sums its dot products in another order (1e-11 relative in FP64, 1e-5 in
+    FP32, as in the fixed-iteration tests above)."""
+    from lfric_core_amd import api
+    from lfric_core_amd.configs import spd_lma
+    from lfric_core_amd.function_space import build_dofmap, colour_cells
+    from lfric_core_amd.rng import Stream
+    from lfric_core_amd.solvers import ConjugateGradient
+    from test_gpu_lma import _limited_area
+    print(f"case cg limited area packed={packed} {dtype.__name__}", flush=True)
+    nl = 5
+    mesh = _limited_area(40)
+    fs, col = build_dofmap(mesh, "W2", nl), colour_cells(mesh)
+    sp = api.Space(ctx, fs)
+    assert sp.plan(col, 0).info()["nclasses"] == 2     # side faces and bottom/top stacks
+    st = Stream(93)
+    M = spd_lma(st, mesh.ncells * nl, 6, 6.0).astype(dtype)
+    b = st.uniform(fs.undf).astype(dtype)
+    xo = np.zeros_like(b)
+    cg_solve(lambda v: oracle.invoke_coloured(0, col, nl, np.zeros_like(v), v, M, fs.dofmap, fs.dofmap), xo, b,
+             max_iter=15, monitor=False)
+    op = api.LMAOperator(torch.from_numpy(M).to(ctx.device), sp, sp, col)
+    if packed:
+        op.packed = api.PackedOperator(op)
+    x = torch.zeros(fs.undf, dtype=op.matrix.dtype, device=ctx.device)
+    res = ConjugateGradient(op, max_iter=15, monitor_convergence=False).apply(x, torch.from_numpy(b).to(ctx.device))
+    assert res.iterations == 15
+    tol = 1e-11 if dtype == np.float64 else 1e-5
+    assert np.linalg.norm(x.cpu().numpy() - xo) <= tol * np.linalg.norm(xo)
