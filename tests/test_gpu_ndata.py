@@ -231,7 +231,7 @@ ABSENT = {
 
 
 @pytest.mark.parametrize("dtype", [np.float32, np.float64])
-@pytest.mark.parametrize("nl", [1, 3])
+@pytest.mark.parametrize("nl", [2, 3])
 @pytest.mark.parametrize("name", list(ABSENT))
 def test_absent_entries_in_bundles_bitexact(ctx, dtype, name, nl):
     """Columns that joined a class of more cells a column, so that whole cells
