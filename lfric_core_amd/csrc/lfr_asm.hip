@@ -507,11 +507,14 @@ k_complex_edge(ComplexOut o, const double* __restrict__ chi1, const double* __re
       }
     double h[6];
 #pragma unroll
-    for (int a = 0; a < 3; ++a)
+    for (int a = 0; a < 3; ++a) {
+      // 1 / detJ on one side first: the square of the cofactors goes with the
+      // fourth power of a length and leaves the range long before H does
+      const double c0 = c[a][0] * idj, c1 = c[a][1] * idj, c2 = c[a][2] * idj;
 #pragma unroll
       for (int b = 0; b <= a; ++b)
-        h[tri_ix(a, b)] =
-            __builtin_fma(c[a][2], c[b][2], __builtin_fma(c[a][1], c[b][1], c[a][0] * c[b][0])) * idj;
+        h[tri_ix(a, b)] = __builtin_fma(c2, c[b][2], __builtin_fma(c1, c[b][1], c0 * c[b][0]));
+    }
 #pragma unroll
     for (int b = 0; b < 12; ++b) {
       double hl[3];   // the column function mapped onto the three axes
