@@ -135,8 +135,8 @@ k_cg_update(T* __restrict__ r, T* __restrict__ z, const T* __restrict__ diag, in
 // not wanted again for a whole iteration, so it streams past the caches
 // (non-temporal) and leaves them to p and r, which the apply and the next
 // update read.  C96L70 solves: FP64 to 1e-10 16.35 -> 15.51 ms (15.89 without
-// the non-temporal x, 15.8 with one stride a trip), refined 9.68 -> 9.63 ms
-// (9.76; 10.4).
+// the non-temporal x, 15.8 with one stride a trip); refined 9.68 and 9.63 ms,
+// no more apart than its runs are (9.76 without, 10.4 with one stride).
 // Every workgroup sums the update's partials in the same order (identical
 // bits); workgroup 0 records the results; S_RZ (read here) is only written
 // by k_cg_alpha.
