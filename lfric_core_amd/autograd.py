@@ -45,7 +45,7 @@ def _zeros(space: "api.Space", dtype):
 
 def _apply(M: torch.Tensor, x: torch.Tensor, op: "api.LMAOperator") -> torch.Tensor:
     op.check_matrix(M)
-    y = torch.empty(op.to_space.undf, dtype=M.dtype, device=M.device)
+    y = M.new_empty(op.to_space.undf)
     if op.to_space.fs.is_discontinuous:
         api._dg_matrix_vector(y, x, M, op)
     else:
@@ -55,7 +55,7 @@ def _apply(M: torch.Tensor, x: torch.Tensor, op: "api.LMAOperator") -> torch.Ten
 
 def _apply_t(M: torch.Tensor, p: torch.Tensor, op: "api.LMAOperator") -> torch.Tensor:
     op.check_matrix(M)
-    b = torch.empty(op.from_space.undf, dtype=M.dtype, device=M.device)
+    b = M.new_empty(op.from_space.undf)
     api._transpose_matrix_vector(b, p, M, op, op.colouring, True)
     return b
 
@@ -64,7 +64,7 @@ def _outer(ybar: torch.Tensor, x: torch.Tensor, op: "api.LMAOperator", out=None,
     """Mbar (+)= alpha * ybar (x) x, per cell-layer (lfr_lma_outer)."""
     acc = out is not None
     if out is None:
-        out = torch.empty(op.matrix.shape, dtype=ybar.dtype, device=ybar.device)
+        out = ybar.new_empty(op.matrix.shape)
     ctx = op.ctx
     ctx.sync_stream()
     check(lib().lfr_lma_outer(ctx.h, api._prec(out), out.data_ptr(), ybar.data_ptr(), x.data_ptr(), op.to_space.h,
