@@ -712,20 +712,23 @@ k_thomas_lanes(T* __restrict__ y, S src, const int32_t* __restrict__ map0, int n
 
 // Whether k_thomas_lanes takes FP64 recurrences of nrow rows: from the mesh
 // size on at which k_thomas_rows no longer holds all columns of 70 rows at
-// once (7 workgroups a CU), as long as k_thomas_lanes does.  µs, k_thomas_rows
-// / k_thomas_lanes, operands in cache: appinv with FP64 pivots on FP32 data
-// C64L70 18.4 / 16.8, C80L70 30.9 / 21.7, C96L20 11.5 / 7.8, C96L30 15.6 / 12.0,
-// C96L50 25.6 / 20.2, C96L70 37.9 / 27.3; tri_solve FP64 C64L70 21.7 / 21.0,
-// C72L70 30.1 / 22.3, C80L70 34.8 / 29.5, C96L70 41.9 / 65.2.  Out of cache: FP64
-// pivots C64L70 18.9 / 20.6, C72L70 20.7 / 20.7, C96L70 39.7 / 36.5, C128L70
-// 57.3 / 65.9; tri_solve C72L70 33.3 / 30.3, C80L70 38.9 / 39.7, C96L70 46.3 /
-// 69.8.  (appinv on FP64 data: C80L70 33.8 / 30.0 in cache, 36.8 / 44.7 out of
-// it: k_thomas_rows.)
+// once (7 workgroups a CU), as long as k_thomas_lanes does (on FP64 data also
+// no more than a wave a SIMD).  µs, k_thomas_rows / k_thomas_lanes, operands in
+// cache: appinv with FP64 pivots on FP32 data C64L70 18.4 / 16.8, C80L70 30.9 /
+// 21.7, C96L20 11.5 / 7.8, C96L30 15.6 / 12.0, C96L50 25.6 / 20.2, C96L70 37.9 /
+// 27.3; on FP64 data C80L20 11.4 / 9.5, C96L20 14.7 / 12.2; tri_solve FP64 C64L70
+// 21.7 / 21.0, C72L70 30.1 / 22.3, C80L70 34.8 / 29.5, C96L70 41.9 / 65.2.  Out of
+// cache: FP64 pivots C64L70 18.9 / 20.6, C72L70 20.7 / 20.7, C96L70 39.7 / 36.5,
+// C128L70 57.3 / 65.9; FP64 data C80L20 12.6 / 12.6, C96L20 15.8 / 16.1, C128L20
+// 23.9 / 25.5; tri_solve C72L70 33.3 / 30.3, C80L70 38.9 / 39.7, C96L70 46.3 / 69.8.
+// (appinv on FP64 data with more rows, C96L30 18.5 / 19.0 in cache and 20.3 / 25.7
+// out of it, C96L50 31.6 / 28.1 and 35.4 / 41.0: k_thomas_rows.)
 template <typename T>
 bool lanes_fit(int ncell, int nrow) {
   constexpr int kCus = 256, kLdsCu = 160 * 1024;
   const int lds = kCols * ((nrow | 1) * 8 + kLanesPitch * (int)sizeof(T) + 4) + nrow * 4;
-  return ncell > kCus * 7 * kRowCols && ncell <= kCus * kCols * (kLdsCu / lds);
+  const int waves = sizeof(T) == 8 ? std::min(4, kLdsCu / lds) : kLdsCu / lds;   // a CU
+  return ncell > kCus * 7 * kRowCols && ncell <= kCus * kCols * waves;
 }
 
 template <typename T, typename C, bool IND, int NROW, typename S>
@@ -820,18 +823,24 @@ int launch_appinv(lfr_ctx* ctx, T* lhs, const T* x, const T* cm, const lfr_space
     }
   }
   const RowsBands<T> src{cm, x, nrow};
-  if constexpr (sizeof(C) > sizeof(T)) {
+  if constexpr (sizeof(C) == 8) {
     if (lanes_fit<T>(ncell, nrow)) {
-      switch (nrow) {   // the row counts of usual layer counts
 #define CASE(NR)                                                           \
   case NR:                                                                 \
     launch_lanes<T, C, true, NR>(ctx->stream, lhs, src, sp, ind, ncell);   \
     LFR_CHECK_LAUNCH(ctx);                                                 \
     return LFR_OK;
-        CASE(20) CASE(21) CASE(30) CASE(31) CASE(50) CASE(51) CASE(70) CASE(71)
-#undef CASE
+      switch (nrow) {   // the row counts of usual layer counts
+        CASE(20) CASE(21)
         default: break;
       }
+      if constexpr (sizeof(T) == 4) {
+        switch (nrow) {
+          CASE(30) CASE(31) CASE(50) CASE(51) CASE(70) CASE(71)
+          default: break;
+        }
+      }
+#undef CASE
     }
   }
   if (!launch_rows<C>(ctx->stream, lhs, src, sp, ind, ncell, nrow)) {

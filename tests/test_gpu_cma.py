@@ -121,19 +121,21 @@ def test_appinv_any_height_bitexact(ctx, dtype, nl):
 
 
 @pytest.mark.parametrize("nl", [19, 20, 21, 30, 31, 50, 51, 70, 71])
-def test_appinv_fp64_pivots_on_large_meshes_bitexact(ctx, nl):
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+def test_appinv_fp64_pivots_on_large_meshes_bitexact(ctx, nl, dtype):
     """29,400 columns (a partial wave at the end): the row counts that have the
-    column-a-lane kernel there and one that has not, a permuted indirection,
-    lhs by itself and in place of x, against the FP64 solve rounded to FP32."""
+    column-a-lane kernel there (20 and 21 in FP64) and some that have not, a
+    permuted indirection, lhs by itself and in place of x; on FP32 data against
+    the FP64 solve rounded to FP32."""
     from lfric_core_amd import api
-    print(f"case appinv FP64 pivots C70 nl={nl}", flush=True)
+    print(f"case appinv FP64 pivots C70 nl={nl} {dtype.__name__}", flush=True)
     m = cubed_sphere(70)
     w3 = build_dofmap(m, "W3", nl)
     st = Stream(39)
-    cm = _helmholtz_columns(st, m.ncells, nl).astype(np.float32)
-    x = st.uniform(w3.undf).astype(np.float32)
+    cm = _helmholtz_columns(st, m.ncells, nl).astype(dtype)
+    x = st.uniform(w3.undf).astype(dtype)
     ind = (np.random.default_rng(7).permutation(nl) + 1).astype(np.int32)
-    ref = oracle.appinv(np.zeros(w3.undf), x.astype(np.float64), cm.astype(np.float64), w3.dofmap, ind).astype(np.float32)
+    ref = oracle.appinv(np.zeros(w3.undf), x.astype(np.float64), cm.astype(np.float64), w3.dofmap, ind).astype(dtype)
     sp = api.Space(ctx, w3)
     op = api.CMAOperator(torch.from_numpy(cm).to(ctx.device), sp, ind)
     xd = torch.from_numpy(x).to(ctx.device)
